@@ -14,17 +14,18 @@
 //    which makes bias, GELU and the store 4-wide.
 //  * bf16 / fp16: v_mfma_f32_16x16x32_bf16 / _f16 (each lane supplies 8
 //    consecutive k); every 16-bit kernel is templated on the input type.
-//    fp32: four v_mfma_f32_16x16x4_f32 per 16-byte fragment; lane group g
-//    supplies k = 4g + j to the j-th MFMA (any consistent permutation of the
-//    k axis leaves the dot product unchanged).
+//    fp32 (element loads only; aligned fp32 problems run gemm_split.hip): four
+//    v_mfma_f32_16x16x4_f32 per 16-byte fragment; lane group g supplies
+//    k = 4g + j to the j-th MFMA (any consistent permutation of the k axis
+//    leaves the dot product unchanged).
 //  * Block (or tile) ids are remapped so that tiles adjacent in the grouped
 //    (GROUP_M) order run on the same XCD (the dispatcher deals block ids
 //    round-robin over the 8 XCDs, each with its own L2).
 //
 // Main loops:
-//  * gemm_kernel: global -> registers -> LDS double buffering (fp32, and small
-//    16-bit problems, any K multiple of 8/4; with element loads, any K, stride
-//    or alignment).
+//  * gemm_kernel: global -> registers -> LDS double buffering (small 16-bit
+//    problems, any K multiple of 8; with element loads, any K, stride or
+//    alignment, fp32 included).
 //  * gemm_pipe_kernel / gemm_pipe_a3_kernel / gemm_slab_kernel: 16-bit
 //    direct-to-LDS multi-stage pipelines, persistent over tiles (see the
 //    comments above them).
@@ -105,8 +106,8 @@ __device__ __forceinline__ void store_block_remap(float* scr, TOut* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Register-staged double-buffered kernel (fp32 and bf16; K % 8 (bf16) or
-// K % 4 (fp32); the K tail of the last 128-byte row is zero-filled).
+// Register-staged double-buffered kernel (K % 8; with element loads any K and
+// fp32 too; the K tail of the last 128-byte row is zero-filled).
 
 template <typename TIn, int BM, int BN, int WGM, int WGN, int EPI, typename TOut, bool EL = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(
@@ -1341,13 +1342,7 @@ static const int kPipeSps[] = {2, 1, 2, 2, 2, 2, 1, 2, 2, 2, 2, 2, 2, 2, 2};
 // Pipelined tiles that also take the residual epilogue (few accumulators a
 // lane, so the tile's old C values fit in registers beside them).
 constexpr int kFirstSmallPipeTile = 17;
-// fp32 configurations (index = tile id for CGPT_F32).
-static const TileCfg kF32Tiles[] = {
-    {128, 128, 2, 2},  // 0
-    {64, 64, 2, 2},    // 1
-};
 constexpr int kNumBf16Tiles = sizeof(kBf16Tiles) / sizeof(kBf16Tiles[0]);
-constexpr int kNumF32Tiles = sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
 
 template <typename TIn, int BM, int BN, int WGM, int WGN, int EPI, typename TOut, bool EL = false>
 static int launch_cfg(const void* a, const void* w, const void* bias, bool bias_bf16, void* c,
@@ -1573,46 +1568,38 @@ static int launch_tile(int tile, const void* a, const void* w, const void* bias,
     return launch_pipe<BM, BN, WGM, WGN, SPS, ST, EPI, TOut, 0, TIn>(a, w, bias, bias_bf16, c, M, \
                                                                      N, K, lda, ldw, ldc,         \
                                                                      vec_store, s);
-  if constexpr (sizeof(TIn) == 2) {
-    switch (tile) {
-      CGPT_GEMM_CASE(0, 256, 256, 2, 2)
-      CGPT_GEMM_CASE(1, 256, 128, 2, 2)
-      CGPT_GEMM_CASE(2, 128, 128, 2, 2)
-      CGPT_GEMM_CASE(3, 128, 64, 2, 2)
-      CGPT_GEMM_CASE(4, 64, 64, 2, 2)
-      CGPT_PIPE_CASE(5, 256, 256, 2, 4, 2, 2)
-      CGPT_PIPE_CASE(6, 256, 256, 2, 4, 1, 4)
-      CGPT_PIPE_CASE(7, 256, 192, 2, 4, 2, 2)
-      CGPT_PIPE_CASE(8, 256, 192, 4, 2, 2, 2)
-      CGPT_PIPE_CASE(9, 256, 128, 4, 2, 2, 3)
-      CGPT_PIPE_CASE(10, 128, 256, 2, 4, 2, 3)
-      CGPT_PIPE_CASE(11, 256, 128, 4, 2, 1, 6)
-      case 12:
-        return launch_pipe_a3<256, 256, 2, 4, EPI, TOut, TIn>(a, w, bias, bias_bf16, c, M, N, K, lda,
-                                                         ldw, ldc, vec_store, s);
-      case 13:
-        return launch_pipe_a3<256, 192, 2, 4, EPI, TOut, TIn>(a, w, bias, bias_bf16, c, M, N, K, lda,
-                                                         ldw, ldc, vec_store, s);
-      case 14:
-        return launch_slab<256, 192, 2, 4, EPI, TOut, TIn>(a, w, bias, bias_bf16, c, M, N, K, lda, ldw,
-                                                      ldc, vec_store, s);
-      case 15:
-        return launch_pipe<256, 256, 2, 4, 2, 2, EPI, TOut, kOutWaveStaged, TIn>(
-            a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
-      case 16:
-        return launch_pipe<256, 256, 2, 4, 2, 2, EPI, TOut, kOutWaveStagedNT, TIn>(
-            a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
-      CGPT_PIPE_CASE(17, 128, 128, 2, 2, 2, 2)
-      CGPT_PIPE_CASE(18, 128, 64, 2, 2, 2, 3)
-      CGPT_PIPE_CASE(19, 64, 64, 2, 2, 2, 3)
-      default: return CGPT_EINVAL;
-    }
-  } else {
-    switch (tile) {
-      CGPT_GEMM_CASE(0, 128, 128, 2, 2)
-      CGPT_GEMM_CASE(1, 64, 64, 2, 2)
-      default: return CGPT_EINVAL;
-    }
+  switch (tile) {
+    CGPT_GEMM_CASE(0, 256, 256, 2, 2)
+    CGPT_GEMM_CASE(1, 256, 128, 2, 2)
+    CGPT_GEMM_CASE(2, 128, 128, 2, 2)
+    CGPT_GEMM_CASE(3, 128, 64, 2, 2)
+    CGPT_GEMM_CASE(4, 64, 64, 2, 2)
+    CGPT_PIPE_CASE(5, 256, 256, 2, 4, 2, 2)
+    CGPT_PIPE_CASE(6, 256, 256, 2, 4, 1, 4)
+    CGPT_PIPE_CASE(7, 256, 192, 2, 4, 2, 2)
+    CGPT_PIPE_CASE(8, 256, 192, 4, 2, 2, 2)
+    CGPT_PIPE_CASE(9, 256, 128, 4, 2, 2, 3)
+    CGPT_PIPE_CASE(10, 128, 256, 2, 4, 2, 3)
+    CGPT_PIPE_CASE(11, 256, 128, 4, 2, 1, 6)
+    case 12:
+      return launch_pipe_a3<256, 256, 2, 4, EPI, TOut, TIn>(a, w, bias, bias_bf16, c, M, N, K, lda,
+                                                       ldw, ldc, vec_store, s);
+    case 13:
+      return launch_pipe_a3<256, 192, 2, 4, EPI, TOut, TIn>(a, w, bias, bias_bf16, c, M, N, K, lda,
+                                                       ldw, ldc, vec_store, s);
+    case 14:
+      return launch_slab<256, 192, 2, 4, EPI, TOut, TIn>(a, w, bias, bias_bf16, c, M, N, K, lda, ldw,
+                                                    ldc, vec_store, s);
+    case 15:
+      return launch_pipe<256, 256, 2, 4, 2, 2, EPI, TOut, kOutWaveStaged, TIn>(
+          a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
+    case 16:
+      return launch_pipe<256, 256, 2, 4, 2, 2, EPI, TOut, kOutWaveStagedNT, TIn>(
+          a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
+    CGPT_PIPE_CASE(17, 128, 128, 2, 2, 2, 2)
+    CGPT_PIPE_CASE(18, 128, 64, 2, 2, 2, 3)
+    CGPT_PIPE_CASE(19, 64, 64, 2, 2, 2, 3)
+    default: return CGPT_EINVAL;
   }
 #undef CGPT_PIPE_CASE
 #undef CGPT_GEMM_CASE
@@ -1640,7 +1627,7 @@ static int small_pipe_tile(int M, int N, int K, int64_t lda, int64_t ldw) {
 // Default tile choice when the caller's table has no entry: the register-staged
 // kernel with the largest tile that still gives every CU about two blocks
 // (128x128 for long K, 128x64 otherwise), smaller tiles for small grids.
-static int auto_tile(bool half, int M, int N, int K, int64_t lda, int64_t ldw, int epi) {
+static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi) {
   // 16-bit (bf16 / fp16) problems with at least one 256x192 tile per CU: the persistent
   // direct-to-LDS pipelines — 256x256 with wave-staged non-temporal stores
   // for wide N (the LM heads) and for the GELU epilogue; 256x192 with
@@ -1650,37 +1637,34 @@ static int auto_tile(bool half, int M, int N, int K, int64_t lda, int64_t ldw, i
   // or 128x256 tile whose last round leaves the fewest CUs idle (ties to the
   // larger tile), as long as it still gives half the CUs a tile; below that
   // the register-staged kernel with smaller tiles.
-  if (half) {
-    auto tiles = [&](int bm, int bn) {
-      return static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-    };
-    const int cus = num_cus();
-    const int64_t t14 = tiles(256, 192);
-    if (t14 >= cus) {
-      const int pick = (N >= 16384 || epi == CGPT_EPI_BIAS_GELU) ? 16 : 14;
-      if (pipe_ok(pick, M, N, K, lda, ldw)) return pick;
-    } else {
-      const int small = small_pipe_tile(M, N, K, lda, ldw);
-      if (small >= 0) return small;
-      const int64_t cand_t[3] = {t14, tiles(256, 128), tiles(128, 256)};
-      const int cand_id[3] = {14, 9, 10};
-      int best = -1;
-      double best_util = 0.0;
-      for (int i = 0; i < 3; ++i) {
-        const int64_t rounds = (cand_t[i] + cus - 1) / cus;
-        const double util = static_cast<double>(cand_t[i]) / static_cast<double>(rounds * cus);
-        if (cand_t[i] * 2 >= cus && util > best_util + 1e-9 && pipe_ok(cand_id[i], M, N, K, lda, ldw)) {
-          best = cand_id[i];
-          best_util = util;
-        }
+  auto tiles = [&](int bm, int bn) {
+    return static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  };
+  const int cus = num_cus();
+  const int64_t t14 = tiles(256, 192);
+  if (t14 >= cus) {
+    const int pick = (N >= 16384 || epi == CGPT_EPI_BIAS_GELU) ? 16 : 14;
+    if (pipe_ok(pick, M, N, K, lda, ldw)) return pick;
+  } else {
+    const int small = small_pipe_tile(M, N, K, lda, ldw);
+    if (small >= 0) return small;
+    const int64_t cand_t[3] = {t14, tiles(256, 128), tiles(128, 256)};
+    const int cand_id[3] = {14, 9, 10};
+    int best = -1;
+    double best_util = 0.0;
+    for (int i = 0; i < 3; ++i) {
+      const int64_t rounds = (cand_t[i] + cus - 1) / cus;
+      const double util = static_cast<double>(cand_t[i]) / static_cast<double>(rounds * cus);
+      if (cand_t[i] * 2 >= cus && util > best_util + 1e-9 && pipe_ok(cand_id[i], M, N, K, lda, ldw)) {
+        best = cand_id[i];
+        best_util = util;
       }
-      if (best >= 0) return best;
     }
+    if (best >= 0) return best;
   }
-  const TileCfg* t = half ? kBf16Tiles : kF32Tiles;
-  const int nt = half ? kNumBf16Tiles : kNumF32Tiles;
-  const int first = half ? (K >= 2048 ? 2 : 3) : 0;
-  const int last = half ? kFirstPipeTile - 1 : nt - 1;
+  const TileCfg* t = kBf16Tiles;
+  const int first = K >= 2048 ? 2 : 3;
+  const int last = kFirstPipeTile - 1;
   for (int i = first; i <= last; ++i) {
     const int64_t blocks =
         static_cast<int64_t>((M + t[i].bm - 1) / t[i].bm) * ((N + t[i].bn - 1) / t[i].bn);
@@ -1721,15 +1705,13 @@ static int launch_resid(int req_tile, const void* a, const void* w, const void* 
                         bool bias_bf16, void* c, int M, int N, int K, int64_t lda, int64_t ldw,
                         int64_t ldc, bool vec_store, hipStream_t s) {
   constexpr int EPI = CGPT_EPI_BIAS_RESID;
-  const int last = sizeof(TIn) == 2 ? kFirstPipeTile - 1 : kNumF32Tiles - 1;
+  const int last = kFirstPipeTile - 1;
   const bool reg_tile = req_tile >= 0 && req_tile <= last;
-  if constexpr (sizeof(TIn) == 2) {
-    if (req_tile >= kFirstSmallPipeTile && req_tile < kNumBf16Tiles &&
-        pipe_ok(req_tile, M, N, K, lda, ldw))
-      return launch_small_pipe<TIn, EPI, TOut>(req_tile, a, w, bias, bias_bf16, c, M, N, K, lda,
-                                               ldw, ldc, vec_store, s);
-  }
-  if constexpr (sizeof(TIn) == 2 && sizeof(TOut) == 4) {
+  if (req_tile >= kFirstSmallPipeTile && req_tile < kNumBf16Tiles &&
+      pipe_ok(req_tile, M, N, K, lda, ldw))
+    return launch_small_pipe<TIn, EPI, TOut>(req_tile, a, w, bias, bias_bf16, c, M, N, K, lda,
+                                             ldw, ldc, vec_store, s);
+  if constexpr (sizeof(TOut) == 4) {
     const int64_t m = M, n = N;
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 191) / 192;
     const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
@@ -1750,14 +1732,12 @@ static int launch_resid(int req_tile, const void* a, const void* w, const void* 
   // Fewer slab tiles than CUs: a 4-wave pipeline tile where K allows it
   // (medium's 4096x512 projections: 13.0 -> 7.8 and 29.2 -> 16.9 us against
   // the 64x64 register tile).
-  if constexpr (sizeof(TIn) == 2) {
-    const int pick = reg_tile ? -1 : small_pipe_tile(M, N, K, lda, ldw);
-    if (pick >= 0)
-      return launch_small_pipe<TIn, EPI, TOut>(pick, a, w, bias, bias_bf16, c, M, N, K, lda, ldw,
-                                               ldc, vec_store, s);
-  }
-  const TileCfg* t = sizeof(TIn) == 2 ? kBf16Tiles : kF32Tiles;
-  const int first = sizeof(TIn) == 2 ? (K >= 2048 ? 2 : 3) : 0;
+  const int pick = reg_tile ? -1 : small_pipe_tile(M, N, K, lda, ldw);
+  if (pick >= 0)
+    return launch_small_pipe<TIn, EPI, TOut>(pick, a, w, bias, bias_bf16, c, M, N, K, lda, ldw,
+                                             ldc, vec_store, s);
+  const TileCfg* t = kBf16Tiles;
+  const int first = K >= 2048 ? 2 : 3;
   int tile = last;
   if (reg_tile) {
     tile = req_tile;
@@ -1774,19 +1754,12 @@ static int launch_resid(int req_tile, const void* a, const void* w, const void* 
   case id:                                                                                        \
     return launch_cfg<TIn, BM, BN, 2, 2, EPI, TOut>(a, w, bias, bias_bf16, c, M, N, K, lda, ldw,  \
                                                      ldc, vec_store, s);
-  if constexpr (sizeof(TIn) == 2) {
-    switch (tile) {
-      CGPT_RES_CFG(0, 256, 256)
-      CGPT_RES_CFG(1, 256, 128)
-      CGPT_RES_CFG(2, 128, 128)
-      CGPT_RES_CFG(3, 128, 64)
-      default: CGPT_RES_CFG(4, 64, 64)
-    }
-  } else {
-    switch (tile) {
-      CGPT_RES_CFG(0, 128, 128)
-      default: CGPT_RES_CFG(1, 64, 64)
-    }
+  switch (tile) {
+    CGPT_RES_CFG(0, 256, 256)
+    CGPT_RES_CFG(1, 256, 128)
+    CGPT_RES_CFG(2, 128, 128)
+    CGPT_RES_CFG(3, 128, 64)
+    default: CGPT_RES_CFG(4, 64, 64)
   }
 #undef CGPT_RES_CFG
 }
@@ -1811,19 +1784,24 @@ static int launch_epi(int epi, int tile, const void* a, const void* w, const voi
     }
 #undef CGPT_EL_CASE
   }
-  switch (epi) {
-    case CGPT_EPI_BIAS_RESID:
-      return launch_resid<TIn, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc,
-                                     vec_store, s);
-    case CGPT_EPI_NONE:
-      return launch_tile<TIn, CGPT_EPI_NONE, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
-    case CGPT_EPI_BIAS:
-      return launch_tile<TIn, CGPT_EPI_BIAS, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
-    case CGPT_EPI_BIAS_GELU:
-      return launch_tile<TIn, CGPT_EPI_BIAS_GELU, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
-    default:
-      return CGPT_EINVAL;
-  }
+  if constexpr (sizeof(TIn) == 4) {
+    return launch_gemm_split(epi, tile, a, w, bias, bias_bf16, c, sizeof(TOut) == 2, M, N, K, lda, ldw,
+                             ldc, vec_store, s);
+  } else {
+    switch (epi) {
+      case CGPT_EPI_BIAS_RESID:
+        return launch_resid<TIn, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc,
+                                       vec_store, s);
+      case CGPT_EPI_NONE:
+        return launch_tile<TIn, CGPT_EPI_NONE, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
+      case CGPT_EPI_BIAS:
+        return launch_tile<TIn, CGPT_EPI_BIAS, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
+      case CGPT_EPI_BIAS_GELU:
+        return launch_tile<TIn, CGPT_EPI_BIAS_GELU, TOut>(tile, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc, vec_store, s);
+      default:
+        return CGPT_EINVAL;
+    }
+    }
 }
 
 }  // namespace cgpt
@@ -1945,8 +1923,11 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
   const int64_t out_align = out16 ? 8 : 16;
   const bool vec_store = (ldc % 4 == 0) && (reinterpret_cast<uintptr_t>(c) % out_align == 0);
   if (tile == CGPT_TILE_SKINNY && (el || f16)) return CGPT_EINVAL;  // vector-rule bf16 / fp32 only
+  // Rows too far apart for the split kernel's 32-bit offsets.
+  const bool f32_far = !bf16 && !f16 && !gemm_split_ok(lda, ldw);
   if (epilogue == CGPT_EPI_BIAS_RESID) {
     if (tile == CGPT_TILE_SKINNY) return CGPT_EINVAL;  // not a skinny epilogue
+    el = el || f32_far;
     // launch_resid picks the kernel (tile: a preference; an id it does not
     // take for these dtypes, in or out of the tile tables, means TILE_AUTO).
     if (el) {
@@ -1966,9 +1947,7 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
       return launch_resid<bf16_t, bf16_t>(tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, s);
     if (bf16)
       return launch_resid<bf16_t, float>(tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, s);
-    if (!out16)
-      return launch_resid<float, float>(tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, s);
-    return launch_resid<float, bf16_t>(tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, s);
+    return launch_gemm_split(epilogue, tile, a, w, bias, bb, c, out16, m, n, k, lda, ldw, ldc, vec_store, s);
   }
   if (tile != CGPT_TILE_AUTO && tile != CGPT_TILE_SKINNY && (tile < 0 || tile >= nt))
     return CGPT_EINVAL;
@@ -1978,8 +1957,9 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
     return launch_gemm_skinny(bf16, epilogue, a, w, bias, bb, c, out16, m, n, k, lda, ldw, ldc,
                               nullptr, 0, nullptr, 0, s);
   }
+  el = el || f32_far;
   if (el) tile = 0;  // the element-load kernel has one tile
-  if (tile == CGPT_TILE_AUTO) tile = auto_tile(bf16 || f16, m, n, k, lda, ldw, epilogue);
+  if (tile == CGPT_TILE_AUTO && (bf16 || f16)) tile = auto_tile(m, n, k, lda, ldw, epilogue);
   if ((bf16 || f16) && tile >= kFirstPipeTile && !pipe_ok(tile, M, N, K, lda, ldw))
     return CGPT_ESHAPE;
   if ((bf16 || f16) && tile >= kFirstPipeTile) {

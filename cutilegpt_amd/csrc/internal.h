@@ -42,4 +42,13 @@ int gemm_partials_split(int M, int N, int K, bool bf16_in);
 int launch_gemm_partials(bool bf16_in, const void* a, const void* w, float* partials, int M, int N,
                          int K, int64_t lda, int64_t ldw, int64_t ldp, int split, hipStream_t s);
 
+// fp32 GEMM on split bf16 operands (gemm_split.hip).  Arguments as cgpt_gemm's,
+// already validated (K, lda and ldw multiples of 4, 16-byte aligned A and W);
+// tile: 0 = 128x128, 1 = 64x64, anything else = by size.
+constexpr int kNumF32Tiles = 2;
+bool gemm_split_ok(int64_t lda, int64_t ldw);  // a tile's rows within 32-bit offsets
+int launch_gemm_split(int epilogue, int tile, const void* a, const void* w, const void* bias,
+                      bool bias_bf16, void* c, bool out_bf16, int M, int N, int K, int64_t lda,
+                      int64_t ldw, int64_t ldc, bool vec_store, hipStream_t s);
+
 }  // namespace cgpt
