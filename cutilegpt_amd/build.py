@@ -42,6 +42,7 @@ def hipcc() -> str:
 # AGPRs (no v_accvgpr_read/write shuttling).
 FILE_FLAGS = {
     "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attention_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

@@ -24,11 +24,12 @@
 //    the second), which leaves the contraction unchanged.
 //  * bf16 / fp16: v_mfma_f32_16x16x32_bf16 / _f16; P is rounded to the input
 //    type before P.V while the normaliser accumulates the unrounded fp32 P.
-//    fp32: v_mfma_f32_16x16x4_f32.
+//    fp32: v_mfma_f32_16x16x4_f32 (head_dim 64: attention_split.hip).
 //  * Softmax runs in the base-2 domain with scale * log2(e) folded into one
 //    multiply; fully masked rows never produce NaN (the running max is clamped
 //    to 0 while it is still -inf).
 #include "common.h"
+#include "internal.h"
 
 namespace cgpt {
 
@@ -722,23 +723,33 @@ static int launch_attn(const void* q, const void* k, const void* v, void* o, int
   const int64_t blocks128 = static_cast<int64_t>(B) * H * ((Tq + 127) / 128);
   const bool small = blocks128 < 4 * static_cast<int64_t>(attn_num_cus());
   const int bq = small ? 64 : 128;
-  const int n_bh = B * H;
-  const int n_qblk = (Tq + bq - 1) / bq;
-  const int64_t blocks = static_cast<int64_t>(n_bh) * n_qblk;
-  if (blocks > 0x7fffffff) return CGPT_ESHAPE;
-  const float scale_log2 = scale * 1.4426950408889634f;
+  // fp32 at head_dim 64: split operands on the bf16 matrix cores, 8x12x512
+  // 50 -> 33 us, 16x12x1024 270 -> 165 (64 queries a block: 195), 1x12x87
+  // 8.9 -> 7.7, against the fp32 MFMA; the error against float64 is below half
+  // of it (8x12x512: 2.8e-7 -> 1.1e-7).  The other head_dims' models are small.
+  if constexpr (sizeof(T) == 4 && HD == 64) {
+    return launch_attention_split(static_cast<const float*>(q), static_cast<const float*>(k),
+                                  static_cast<const float*>(v), static_cast<float*>(o), B, H, Tq, Tk, st,
+                                  scale, causal, bq, s);
+  } else {
+    const int n_bh = B * H;
+    const int n_qblk = (Tq + bq - 1) / bq;
+    const int64_t blocks = static_cast<int64_t>(n_bh) * n_qblk;
+    if (blocks > 0x7fffffff) return CGPT_ESHAPE;
+    const float scale_log2 = scale * 1.4426950408889634f;
 #define CGPT_ATTN_LAUNCH(QTW)                                                                     \
-  hipLaunchKernelGGL((attn_fwd_kernel<T, HD, QTW>), dim3(static_cast<unsigned>(blocks)),            \
-                     dim3(kAttnThreads), 0, s, static_cast<const T*>(q), static_cast<const T*>(k), \
-                     static_cast<const T*>(v), static_cast<T*>(o), H, Tq, Tk, st[0], st[1], st[2], \
-                     st[3], st[4], st[5], st[6], st[7], st[8], st[9], st[10], st[11], scale_log2, \
-                     causal, n_bh)
-  if (small)
-    CGPT_ATTN_LAUNCH(1);
-  else
-    CGPT_ATTN_LAUNCH(2);
+    hipLaunchKernelGGL((attn_fwd_kernel<T, HD, QTW>), dim3(static_cast<unsigned>(blocks)),            \
+                       dim3(kAttnThreads), 0, s, static_cast<const T*>(q), static_cast<const T*>(k), \
+                       static_cast<const T*>(v), static_cast<T*>(o), H, Tq, Tk, st[0], st[1], st[2], \
+                       st[3], st[4], st[5], st[6], st[7], st[8], st[9], st[10], st[11], scale_log2, \
+                       causal, n_bh)
+    if (small)
+      CGPT_ATTN_LAUNCH(1);
+    else
+      CGPT_ATTN_LAUNCH(2);
 #undef CGPT_ATTN_LAUNCH
-  return hip_status(hipGetLastError());
+    return hip_status(hipGetLastError());
+  }
 }
 
 template <typename T>

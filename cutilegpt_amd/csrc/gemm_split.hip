@@ -21,6 +21,7 @@
 #include "common.h"
 #include "gemm_common.h"
 #include "internal.h"
+#include "split.h"
 
 namespace cgpt {
 
@@ -28,18 +29,6 @@ namespace cgpt {
 __device__ __forceinline__ void mfma32(const u32x4_t& a, const u32x4_t& b, f32x16_t& c) {
   c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
                                               __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
-// Four fp32 values into four bf16 values of each plane.
-__device__ __forceinline__ void split3(const u32x4_t& v, u32x2_t& h, u32x2_t& m, u32x2_t& l) {
-#pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const float a = __uint_as_float(v[2 * p]), b = __uint_as_float(v[2 * p + 1]);
-    h[p] = pack_bf16x2(a, b);
-    const float ra = a - __uint_as_float(h[p] << 16), rb = b - __uint_as_float(h[p] & 0xffff0000u);
-    m[p] = pack_bf16x2(ra, rb);
-    l[p] = pack_bf16x2(ra - __uint_as_float(m[p] << 16), rb - __uint_as_float(m[p] & 0xffff0000u));
-  }
 }
 #endif
 
@@ -191,13 +180,12 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
       for (int j = 0; j < TN; ++j) wf[p][j] = *reinterpret_cast<const u32x4_t*>(sw + p * W_PLANE + j * 512);
     }
     put_all(d, (it + 1) * KG + grp, buf ^ 1, (it + 1 + PD) * KG + grp, whole);
-    constexpr int kPw[6] = {0, 0, 1, 1, 0, 2}, kPa[6] = {0, 1, 0, 1, 2, 0};
 #pragma unroll
     for (int t = 0; t < 6; ++t)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) mfma32(wf[kPw[t]][j], af[kPa[t]][i], acc[i][j]);
+        for (int j = 0; j < TN; ++j) mfma32(wf[kSplitA[t]][j], af[kSplitB[t]][i], acc[i][j]);
     stage_sync();
   };
   if constexpr (PD == 1) {
@@ -253,7 +241,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
   auto check_row = [&](uint32_t v) {
     v |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kDppXor1, 0xF, 0xF, true));
     v |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kDppXor2, 0xF, 0xF, true));
-    tiny = tiny || ((v & 0x7fffffffu) != 0 && (v & 0x70000000u) == 0);
+    tiny = tiny || ((v & 0x7fffffffu) != 0 && (v & kSplitNormalBits) == 0);
   };
 #pragma unroll
   for (int i = 0; i < A_LD; ++i) check_row(oa[i]);

@@ -51,4 +51,11 @@ int launch_gemm_split(int epilogue, int tile, const void* a, const void* w, cons
                       bool bias_bf16, void* c, bool out_bf16, int M, int N, int K, int64_t lda,
                       int64_t ldw, int64_t ldc, bool vec_store, hipStream_t s);
 
+// Attention forward for fp32 inputs of head_dim 64 on split bf16 operands
+// (attention_split.hip); arguments as cgpt_attention_fwd's, already validated,
+// st its twelve strides, queries a block 64 or 128.
+int launch_attention_split(const float* q, const float* k, const float* v, float* o, int B, int H,
+                           int Tq, int Tk, const int64_t* st, float scale, int causal, int queries,
+                           hipStream_t s);
+
 }  // namespace cgpt
