@@ -1362,7 +1362,7 @@ static int launch_cfg(const void* a, const void* w, const void* bias, bool bias_
 // Compute units of the current device (persistent grids launch as many blocks
 // per CU as fit).  Cached per device id; concurrent first calls store the same
 // value.
-static int num_cus() {
+int num_cus() {
   static std::atomic<int> cache[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
@@ -1605,63 +1605,90 @@ static int launch_tile(int tile, const void* a, const void* w, const void* bias,
 #undef CGPT_GEMM_CASE
 }
 
-// The largest 4-wave pipeline tile that gives the CUs at least 1.5 tiles each
-// (their blocks run two or three a CU), else 64x64; -1 when K or the offsets
-// rule the pipeline out.  Residual projections measured with each: XL
-// 4096 x 1600 x 6400 128x128 91 / 128x64 112 / 64x64 138 us, 4096 x 1600 x
-// 1600 33 / 38 / 41 us (the slab's 144 tiles: 123 and 43 us); medium
-// 4096 x 512 x 2048 26 / 20 / 17 us.
-static int small_pipe_tile(int M, int N, int K, int64_t lda, int64_t ldw) {
-  constexpr int kIds[3] = {17, 18, 19}, kBm[3] = {128, 128, 64}, kBn[3] = {128, 64, 64};
-  const int64_t cus = num_cus();
-  int fallback = -1;
-  for (int i = 0; i < 3; ++i) {
-    if (!pipe_ok(kIds[i], M, N, K, lda, ldw)) continue;
-    const int64_t t = static_cast<int64_t>((M + kBm[i] - 1) / kBm[i]) * ((N + kBn[i] - 1) / kBn[i]);
-    if (2 * t >= 3 * cus) return kIds[i];
-    fallback = kIds[i];
-  }
-  return fallback;
+// Default tile choice for 16-bit problems (no entry in the caller's table): the
+// tile whose predicted launch time is lowest.
+//
+// A tile's time is modelled as
+//     start + rounds + fill * (bytes into LDS) + out * M N + gelu * M N + ops * (operand bytes)
+// where a round is one set of blocks as the CUs hold them: with j blocks a CU it
+// costs step[j] for every k64 step and end[j] once; all rounds but the last have
+// `blocks` a CU.  The coefficients (us, us per MB and per 2^20 elements / 10^6)
+// are a least-squares fit to 450 problems (M 70 to 16 384; the four layer
+// products at d = 256 to 1600; bias, GELU and residual epilogues) timed with
+// every tile over operands rotated past the caches.  The model's pick takes
+// 1.002 times the best tile's time in the geometric mean over them (1.12 at
+// most); the choice it replaces (tiles counted per CU) took 1.22 (2.44), mostly
+// where few tiles leave the CUs waiting: 70 x 1600 x 6400 36.4 -> 14.9 us,
+// 591 x 2304 x 768 8.9 -> 8.4, 2700 x 768 x 3072 39 -> 26, 4096 x 2304 x 768
+// 26 -> 19.3, 4096 x 768 x 3072 with the residual 43 -> 33.
+struct TileCost {
+  int id, bm, bn, blocks;
+  float start, step[3], end[3], fill, out, gelu, ops;
+};
+constexpr int kFirstKgroupTile = 100;  // internal ids: gemm_kgroup.hip's tiles
+static const TileCost kTileCosts[] = {
+    {14, 256, 192, 1, 2.247f, {0.984f}, {3.668f}, 0.0056f, 0.f, 0.299f, 0.152f},
+    {16, 256, 256, 1, 0.279f, {1.255f}, {5.920f}, 0.0091f, 0.f, 0.275f, 0.094f},
+    {17, 128, 128, 2, 5.032f, {0.613f, 0.670f}, {0.f, 1.975f}, 0.0129f, 0.0709f, 0.0027f, 0.0772f},
+    {18, 128, 64, 2, 4.410f, {0.385f, 0.499f}, {0.f, 0.567f}, 0.0088f, 0.0687f, 0.0069f, 0.0831f},
+    {19, 64, 64, 3, 3.865f, {0.267f, 0.343f, 0.518f}, {0.f, 0.138f, 0.657f}, 0.0056f, 0.0494f, 0.f, 0.0881f},
+    {100, 32, 32, 1, 1.963f, {0.079f}, {1.849f}, 0.0121f, 0.1237f, 0.349f, 0.0227f},
+    {101, 64, 32, 1, 2.134f, {0.116f}, {1.870f}, 0.0129f, 0.0610f, 0.384f, 0.f},
+    {102, 64, 64, 1, 2.264f, {0.185f}, {1.614f}, 0.0117f, 0.0483f, 0.128f, 0.0263f},
+    {103, 64, 96, 1, 2.575f, {0.228f}, {1.849f}, 0.0116f, 0.0518f, 0.0788f, 0.0374f},
+    {104, 96, 96, 1, 2.950f, {0.290f}, {2.195f}, 0.0103f, 0.0789f, 0.0723f, 0.0198f},
+    {105, 128, 96, 1, 2.632f, {0.420f}, {2.353f}, 0.0083f, 0.0724f, 0.0510f, 0.0363f},
+    {106, 128, 128, 1, 2.804f, {0.498f}, {2.752f}, 0.0057f, 0.0900f, 0.0302f, 0.0353f},
+    {107, 192, 96, 1, 2.883f, {0.568f}, {2.941f}, 0.0053f, 0.0923f, 0.0440f, 0.0253f},
+};
+// The slab kernel with its residual ring (tile 14, residual epilogue).
+static const TileCost kSlabResidCost = {14, 256, 192, 1, 0.f, {1.222f}, {0.f}, 0.0014f, 0.1194f, 0.f, 0.1617f};
+
+static float tile_cost(const TileCost& t, uint32_t M, uint32_t N, float k64, float mn, float ops_mb, int epi,
+                       uint32_t cus) {
+  const uint64_t tiles = static_cast<uint64_t>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+  const uint32_t q = tiles < 0xffffffffu ? static_cast<uint32_t>(tiles) : 0xffffffffu;
+  const uint32_t slots = cus * t.blocks, full = q / slots, last = q - full * slots;
+  const int rest = last == 0 ? 0 : last <= cus ? 1 : last <= 2 * cus ? 2 : 3;  // last round's blocks a CU
+  float us = t.start + static_cast<float>(full) * (k64 * t.step[t.blocks - 1] + t.end[t.blocks - 1]);
+  if (rest > 0) us += k64 * t.step[rest - 1] + t.end[rest - 1];
+  us += t.fill * static_cast<float>(q) * static_cast<float>(t.bm + t.bn) * k64 * 128e-6f;
+  us += t.out * mn * (epi == CGPT_EPI_BIAS_RESID ? 12.f : 2.f);
+  if (epi == CGPT_EPI_BIAS_GELU) us += t.gelu * mn;
+  return us + t.ops * ops_mb;
 }
 
-// Default tile choice when the caller's table has no entry: the register-staged
-// kernel with the largest tile that still gives every CU about two blocks
-// (128x128 for long K, 128x64 otherwise), smaller tiles for small grids.
-static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi) {
-  // 16-bit (bf16 / fp16) problems with at least one 256x192 tile per CU: the persistent
-  // direct-to-LDS pipelines — 256x256 with wave-staged non-temporal stores
-  // for wide N (the LM heads) and for the GELU epilogue; 256x192 with
-  // block-staged stores otherwise.  With fewer tiles than CUs, a 4-wave
-  // pipeline tile (several blocks a CU; medium's 4096 x 2048 x 512 c_fc:
-  // 15.7 us against 17.3 for 256x128), else the persistent 256x192, 256x128
-  // or 128x256 tile whose last round leaves the fewest CUs idle (ties to the
-  // larger tile), as long as it still gives half the CUs a tile; below that
-  // the register-staged kernel with smaller tiles.
-  auto tiles = [&](int bm, int bn) {
-    return static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-  };
-  const int cus = num_cus();
-  const int64_t t14 = tiles(256, 192);
-  if (t14 >= cus) {
-    const int pick = (N >= 16384 || epi == CGPT_EPI_BIAS_GELU) ? 16 : 14;
-    if (pipe_ok(pick, M, N, K, lda, ldw)) return pick;
-  } else {
-    const int small = small_pipe_tile(M, N, K, lda, ldw);
-    if (small >= 0) return small;
-    const int64_t cand_t[3] = {t14, tiles(256, 128), tiles(128, 256)};
-    const int cand_id[3] = {14, 9, 10};
-    int best = -1;
-    double best_util = 0.0;
-    for (int i = 0; i < 3; ++i) {
-      const int64_t rounds = (cand_t[i] + cus - 1) / cus;
-      const double util = static_cast<double>(cand_t[i]) / static_cast<double>(rounds * cus);
-      if (cand_t[i] * 2 >= cus && util > best_util + 1e-9 && pipe_ok(cand_id[i], M, N, K, lda, ldw)) {
-        best = cand_id[i];
-        best_util = util;
-      }
+// The cheapest tile that takes the problem; -1 when none does (K % 64 != 0, or
+// operands past the pipelines' 32-bit offsets).  kgroup, slab: whether
+// gemm_kgroup.hip's tiles and (residual epilogue) the slab kernel take it.
+static int cheapest_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, bool kgroup, bool slab) {
+  const bool resid = epi == CGPT_EPI_BIAS_RESID;
+  const uint32_t cus = num_cus(), m = M, n = N;
+  const float k64 = static_cast<float>(K) / 64, mn = static_cast<float>(M) * static_cast<float>(N) * 1e-6f;
+  const float ops_mb = (static_cast<float>(M) + static_cast<float>(N)) * static_cast<float>(K) * 2e-6f;
+  int best = -1;
+  float best_us = 0.f;
+  for (const TileCost& t : kTileCosts) {
+    if (t.id >= kFirstKgroupTile ? !kgroup : !pipe_ok(t.id, M, N, K, lda, ldw)) continue;
+    if (resid && (t.id == 16 || (t.id == 14 && !slab))) continue;
+    const float us = tile_cost(resid && t.id == 14 ? kSlabResidCost : t, m, n, k64, mn, ops_mb, epi, cus);
+    if (best < 0 || us < best_us) {
+      best = t.id;
+      best_us = us;
     }
-    if (best >= 0) return best;
   }
+  return best;
+}
+
+// Without the residual epilogue.  Wide N (the LM heads) with a 256x192 tile for
+// every CU: 256x256 with wave-staged non-temporal stores.  Problems no
+// pipelined kernel takes: the register-staged kernel with the largest tile that
+// still gives every CU about two blocks (128x128 for long K, 128x64 otherwise).
+static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, bool kgroup) {
+  const int64_t t14 = static_cast<int64_t>((M + 255) / 256) * ((N + 191) / 192);
+  if (N >= 16384 && t14 >= num_cus() && pipe_ok(16, M, N, K, lda, ldw)) return 16;
+  const int pick = cheapest_tile(M, N, K, lda, ldw, epi, kgroup, true);
+  if (pick >= 0) return pick;
   const TileCfg* t = kBf16Tiles;
   const int first = K >= 2048 ? 2 : 3;
   const int last = kFirstPipeTile - 1;
@@ -1676,13 +1703,10 @@ static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi) {
 // Residual epilogue (C += A W^T + bias).  `tile`: 14 = the slab kernel's
 // residual ring (16-bit inputs into fp32 C, at least 8 k64 steps, whole
 // 4-column groups, 32-bit offsets; otherwise as TILE_AUTO); 17-19 = that
-// small pipeline tile (16-bit inputs, K % 64 == 0; otherwise as TILE_AUTO); a
-// register-staged tile id (bf16 / fp16 0-4, fp32 0-1) = that tile; anything
-// else = TILE_AUTO: the slab kernel when its 256x192 tiles give every CU a
-// tile, else the largest 4-wave pipeline tile (128x128, 128x64, 64x64) with
-// at least 1.5 tiles a CU, else 64x64 (16-bit inputs, K % 64 == 0), else the
-// register-staged tile the library's heuristic gives (the largest with 512
-// blocks, 64x64 below that).
+// small pipeline tile (K % 64 == 0; otherwise as TILE_AUTO); a register-staged
+// tile id (0-4) = that tile; anything else = TILE_AUTO: the cheapest of the
+// tiles with this epilogue (cheapest_tile), else the register-staged tile the
+// library's heuristic gives (the largest with 512 blocks, 64x64 below that).
 template <typename TIn, int EPI, typename TOut>
 static int launch_small_pipe(int tile, const void* a, const void* w, const void* bias,
                              bool bias_bf16, void* c, int M, int N, int K, int64_t lda,
@@ -1711,16 +1735,20 @@ static int launch_resid(int req_tile, const void* a, const void* w, const void* 
       pipe_ok(req_tile, M, N, K, lda, ldw))
     return launch_small_pipe<TIn, EPI, TOut>(req_tile, a, w, bias, bias_bf16, c, M, N, K, lda,
                                              ldw, ldc, vec_store, s);
+  const int64_t m = M, n = N;
+  const int tiles_m = (M + 255) / 256, tiles_n = (N + 191) / 192;
+  const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
+  const bool slab = sizeof(TOut) == 4 && K % 64 == 0 && K / 64 >= kResidMinSteps && n % 4 == 0 &&
+                    ldc % 4 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0 &&
+                    (m + 256) * ldc * 4 < (int64_t{1} << 32) && (m + 256) * lda * 2 < (int64_t{1} << 32) &&
+                    (n + 192) * ldw * 2 < (int64_t{1} << 32) && 256 * ldc * 4 < 0x7fffffff &&
+                    tiles <= 0x7fffffff;
+  int pick = req_tile;
+  if (!reg_tile && !(req_tile == 14 && slab))
+    pick = cheapest_tile(M, N, K, lda, ldw, EPI,
+                         gemm_kgroup_ok(M, N, K, lda, ldw, ldc, c, sizeof(TOut) == 2), slab);
   if constexpr (sizeof(TOut) == 4) {
-    const int64_t m = M, n = N;
-    const int tiles_m = (M + 255) / 256, tiles_n = (N + 191) / 192;
-    const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
-    const bool want = req_tile == 14 || (!reg_tile && tiles >= num_cus());
-    if (want && K % 64 == 0 && K / 64 >= kResidMinSteps && n % 4 == 0 && ldc % 4 == 0 &&
-        reinterpret_cast<uintptr_t>(c) % 16 == 0 && (m + 256) * ldc * 4 < (int64_t{1} << 32) &&
-        (m + 256) * lda * 2 < (int64_t{1} << 32) && (n + 192) * ldw * 2 < (int64_t{1} << 32) &&
-        256 * ldc * 4 < 0x7fffffff) {
-      if (tiles > 0x7fffffff) return CGPT_ESHAPE;
+    if (pick == 14) {
       const int grid = static_cast<int>(tiles < num_cus() ? tiles : num_cus());
       hipLaunchKernelGGL((gemm_slab_kernel<256, 192, 2, 4, EPI, float, TIn>), dim3(grid), dim3(512),
                          0, s, static_cast<const TIn*>(a), static_cast<const TIn*>(w), bias,
@@ -1729,13 +1757,12 @@ static int launch_resid(int req_tile, const void* a, const void* w, const void* 
       return hip_status(hipGetLastError());
     }
   }
-  // Fewer slab tiles than CUs: a 4-wave pipeline tile where K allows it
-  // (medium's 4096x512 projections: 13.0 -> 7.8 and 29.2 -> 16.9 us against
-  // the 64x64 register tile).
-  const int pick = reg_tile ? -1 : small_pipe_tile(M, N, K, lda, ldw);
-  if (pick >= 0)
-    return launch_small_pipe<TIn, EPI, TOut>(pick, a, w, bias, bias_bf16, c, M, N, K, lda, ldw,
-                                             ldc, vec_store, s);
+  if (pick >= kFirstKgroupTile)
+    return launch_gemm_kgroup(std::is_same<TIn, f16_t>::value, EPI, pick - kFirstKgroupTile, a, w, bias,
+                              bias_bf16, c, sizeof(TOut) == 2, M, N, K, lda, ldw, ldc, s);
+  if (pick >= kFirstSmallPipeTile)
+    return launch_small_pipe<TIn, EPI, TOut>(pick, a, w, bias, bias_bf16, c, M, N, K, lda, ldw, ldc,
+                                             vec_store, s);
   const TileCfg* t = kBf16Tiles;
   const int first = K >= 2048 ? 2 : 3;
   int tile = last;
@@ -1959,7 +1986,12 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
   }
   el = el || f32_far;
   if (el) tile = 0;  // the element-load kernel has one tile
-  if (tile == CGPT_TILE_AUTO && (bf16 || f16)) tile = auto_tile(m, n, k, lda, ldw, epilogue);
+  if (tile == CGPT_TILE_AUTO && (bf16 || f16)) {
+    tile = auto_tile(m, n, k, lda, ldw, epilogue, gemm_kgroup_ok(M, N, K, lda, ldw, ldc, c, out16));
+    if (tile >= kFirstKgroupTile)
+      return launch_gemm_kgroup(f16, epilogue, tile - kFirstKgroupTile, a, w, bias, bb, c, out16, m, n, k,
+                                lda, ldw, ldc, s);
+  }
   if ((bf16 || f16) && tile >= kFirstPipeTile && !pipe_ok(tile, M, N, K, lda, ldw))
     return CGPT_ESHAPE;
   if ((bf16 || f16) && tile >= kFirstPipeTile) {

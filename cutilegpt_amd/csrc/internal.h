@@ -6,6 +6,9 @@
 
 namespace cgpt {
 
+// Compute units of the current device.
+int num_cus();
+
 // Argument checks shared by the GEMM entry points (cgpt_gemm, the skinny
 // variants): CGPT_OK when the problem is well formed, M == 0 or N == 0
 // included (nothing to launch).  Without `elem_loads` (the skinny kernels)
@@ -50,6 +53,15 @@ bool gemm_split_ok(int64_t lda, int64_t ldw);  // a tile's rows within 32-bit of
 int launch_gemm_split(int epilogue, int tile, const void* a, const void* w, const void* bias,
                       bool bias_bf16, void* c, bool out_bf16, int M, int N, int K, int64_t lda,
                       int64_t ldw, int64_t ldc, bool vec_store, hipStream_t s);
+
+// 16-bit GEMM of few output tiles (gemm_kgroup.hip).  Arguments as cgpt_gemm's,
+// already validated, a problem for which gemm_kgroup_ok holds; tile 0..7.
+constexpr int kNumKgroupTiles = 8;
+bool gemm_kgroup_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t ldc, const void* c,
+                    bool out16);
+int launch_gemm_kgroup(bool f16, int epilogue, int tile, const void* a, const void* w, const void* bias,
+                       bool bias_half, void* c, bool out16, int M, int N, int K, int64_t lda, int64_t ldw,
+                       int64_t ldc, hipStream_t s);
 
 // Attention forward for fp32 inputs of head_dim 64 on split bf16 operands
 // (attention_split.hip); arguments as cgpt_attention_fwd's, already validated,

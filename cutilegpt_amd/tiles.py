@@ -34,17 +34,17 @@ Tile ids index the configuration table compiled into libcgpt.so
     residual epilogue; problems whose 256x192 tiles would leave CUs idle),
     launched with as many blocks as fit a CU (two, or three at 64x64):
           17 = 128x128 (2 stages)  18 = 128x64 (3 stages)  19 = 64x64 (3 stages)
-    fp32: 0 = 128x128, 1 = 64x64
+    fp32 (split bf16 operands, csrc/gemm_split.hip): 0 = 128x128, 1 = 64x64
 
-``TABLE`` maps (dtype, M bucket, N, K) to the tile that won a sweep of every
-tile on MI355X (``python -m cutilegpt_amd.tune``: each model's prefill GEMMs,
-bias / GELU / residual epilogues and output types as the forward runs them).
-The M bucket is the power of two at or above M, so one entry covers every M
-in (bucket / 2, bucket] — batch x sequence products that differ a little share
-a choice.  Anything else falls back to the library's own heuristic
-(``TILE_AUTO``: the persistent tile that fills the 256 CUs best, else the
-register-staged kernel's largest tile giving every CU about two blocks).  For
-the residual epilogue (attn / MLP c_proj into the fp32 residual stream) a
+``TABLE`` maps (dtype, M bucket, N, K) to a tile (``python -m cutilegpt_amd.tune``
+sweeps every tile over each model's prefill GEMMs).  The M bucket is the power
+of two at or above M, so one entry covers every M in (bucket / 2, bucket].
+Anything else takes the library's own choice (``TILE_AUTO``): for 16-bit inputs
+the tile whose predicted launch time is lowest (``tile_cost`` in
+``csrc/gemm.hip``; the tiles of ``csrc/gemm_kgroup.hip``, which have no id here,
+among them), for the exact M rather than its bucket, which is why the table
+holds only the LM heads and products whose best tile is the same over a bucket.
+For the residual epilogue (attn / MLP c_proj into the fp32 residual stream) a
 tile id picks between the slab kernel (14), the small pipeline tiles (17-19)
 and the register-staged tiles.
 """
@@ -67,21 +67,11 @@ _B = _lib.CGPT_BF16
 TABLE: Dict[Tuple[int, int, int, int], int] = {
     # GPT-2 124M prefill, M = 16 x 1024
     (_B, 16384, 2304, 768): 14,   # c_attn       1075
-    (_B, 16384, 768, 768): 14,    # attn c_proj   636
-    (_B, 16384, 3072, 768): 16,   # c_fc + GELU  1074
-    (_B, 16384, 768, 3072): 14,   # mlp c_proj   1056
     (_B, 16384, 50304, 768): 16,  # lm head (vocab padded), fp32 out  1015
     # 'medium' (8 layers, d 512) prefill, M = 16 x 256
-    (_B, 4096, 1536, 512): 14,    # c_attn        474
     (_B, 4096, 512, 512): 19,     # attn c_proj   266 (64x64 pipeline)
-    (_B, 4096, 2048, 512): 17,    # c_fc + GELU   580 (128x128 pipeline)
-    (_B, 4096, 512, 2048): 19,    # mlp c_proj    497 (64x64 pipeline)
     (_B, 4096, 50304, 512): 16,   # lm head       877
     # GPT-2 XL (48 layers, d 1600) prefill inside generate, M = 32 x 128
-    (_B, 4096, 4800, 1600): 14,   # c_attn       1015
-    (_B, 4096, 1600, 1600): 17,   # attn c_proj   661 (128x128 pipeline; slab: 144 tiles)
-    (_B, 4096, 6400, 1600): 16,   # c_fc + GELU   997 (128x128 pipeline 968)
-    (_B, 4096, 1600, 6400): 17,   # mlp c_proj    934 (128x128 pipeline)
     (_B, 4096, 50304, 1600): 16,  # lm head      1156
 }
 

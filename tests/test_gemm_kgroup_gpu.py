@@ -1,0 +1,76 @@
+"""16-bit GEMM with K shared between wave groups (csrc/gemm_kgroup.hip), as
+TILE_AUTO picks it for problems of few tiles, against float64.
+
+Shapes: for each of its tiles the edges of rows and columns, K of one k64 stage
+(fewer than the groups), a stage count the groups do not divide, and the largest
+M of the tile's range."""
+
+import math
+
+import pytest
+import torch
+
+from cutilegpt_amd import _lib
+
+pytestmark = pytest.mark.gpu
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+CODE = {BF16: _lib.CGPT_BF16, F16: _lib.CGPT_F16, F32: _lib.CGPT_F32}
+
+SHAPES = [
+    (65, 36, 64), (70, 100, 128), (97, 768, 3072), (130, 260, 192),   # 32x32, 4 groups
+    (300, 900, 320), (591, 768, 3072),                                # 64x32, 4 groups
+    (1000, 768, 768), (1100, 772, 1088),                              # 64x64, 2 groups
+    (1500, 768, 3072),                                                # 64x96, 2 groups
+    (2700, 768, 768), (2690, 764, 832),                               # 96x96, 2 groups
+    (2900, 772, 704), (3300, 768, 3072),                              # 128x96
+    (2048, 1600, 6400), (4001, 772, 1088),                            # 128x128
+    (6000, 768, 3072),                                                # 192x96
+]
+
+
+def gemm(gpu, a, w, b, epi, out, bias_dtype=None):
+    m, k = a.shape
+    n = w.shape[0]
+    b = b.to(bias_dtype or a.dtype)
+    _lib.check(_lib.load().cgpt_gemm(
+        a.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k, a.stride(0), w.stride(0),
+        out.stride(0), CODE[a.dtype], CODE[b.dtype], CODE[out.dtype], epi, _lib.TILE_AUTO,
+        torch.cuda.current_stream(gpu).cuda_stream), "gemm")
+    return out
+
+
+def problem(gpu, m, n, k, dtype):
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    a = torch.randn(m, k, device=gpu, generator=g).to(dtype)
+    w = (torch.randn(n, k, device=gpu, generator=g) * 0.05).to(dtype)
+    b = torch.randn(n, device=gpu, generator=g).to(dtype)
+    return a, w, b, a.double() @ w.double().t() + b.double()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_kgroup_shapes(gpu, m, n, k, dtype):
+    a, w, b, ref = problem(gpu, m, n, k, dtype)
+    # fp32 sums of K products of |a w| ~ 0.05, as for the other tiles
+    tol = 1e-4 * math.sqrt(k / 64)
+    out = torch.full((m, n + 4), 7.0, dtype=F32, device=gpu)
+    gemm(gpu, a, w, b, _lib.EPI_BIAS, out[:, :n], F32 if m % 2 else None)
+    assert (out[:, :n].double() - ref).abs().max() <= tol + 1e-5 * ref.abs().max()
+    assert (out[:, n:] == 7.0).all()  # padding of the rows untouched
+    x = torch.randn(m, n, device=gpu) * 4
+    out = gemm(gpu, a, w, b, _lib.EPI_BIAS_RESID, x.clone())
+    assert (out.double() - ref - x.double()).abs().max() <= 2 * tol
+    half = gemm(gpu, a, w, b, _lib.EPI_BIAS_GELU, torch.empty(m, n, dtype=dtype, device=gpu))
+    want = torch.nn.functional.gelu(ref, approximate="tanh")
+    eps = 2.0 ** -8 if dtype == BF16 else 2.0 ** -11
+    assert ((half.double() - want).abs() <= eps * want.abs() + tol + 1e-4).all()
+    half = x.to(dtype)
+    want = ref + half.double()
+    gemm(gpu, a, w, b, _lib.EPI_BIAS_RESID, half)
+    assert ((half.double() - want).abs() <= eps * want.abs() + 2 * tol).all()
+
+
+def test_kgroup_repeats_bit_for_bit(gpu):
+    a, w, b, _ = problem(gpu, 97, 768, 3072, BF16)
+    outs = [gemm(gpu, a, w, b, _lib.EPI_BIAS, torch.empty(97, 768, device=gpu)) for _ in range(3)]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
