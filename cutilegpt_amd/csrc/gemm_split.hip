@@ -117,27 +117,22 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
     *reinterpret_cast<u32x2_t*>(p + 2 * plane) = l;
   };
   uint8_t* const gbase = smem + grp * 2 * STAGE;
-  // Stage kt from register set d into buffer `buf`, each register reloaded
-  // with stage `next` as it is freed.  `whole`: kt * BK + BK <= K is known.
-  auto put_all = [&](int d, int kt, int buf, int next, bool whole) {
-    if (!whole) {
-      const bool live = kt * BK + kq * 4 < K;
-#pragma unroll
-      for (int i = 0; i < A_LD; ++i) ra[d][i] = live ? ra[d][i] : u32x4_t{0, 0, 0, 0};
-#pragma unroll
-      for (int i = 0; i < W_LD; ++i) rw[d][i] = live ? rw[d][i] : u32x4_t{0, 0, 0, 0};
-    }
-    const uint32_t ko = koff(next);
+  // Chunk c (A's, then W's) of stage kt from register set d into buffer `buf`,
+  // its register reloaded with the stage at `ko`.  `whole`: the stage is known
+  // to end within K.
+  constexpr int NCH = A_LD + W_LD;
+  auto put_chunk = [&](int c, int d, int kt, int buf, uint32_t ko, bool whole) {
+    const bool live = whole || kt * BK + kq * 4 < K;
     uint8_t* sa = gbase + buf * STAGE;
-#pragma unroll
-    for (int i = 0; i < A_LD; ++i) {
-      put(sa, A_RUN, A_PLANE, (tid + i * NT) / QPR, ra[d][i], oa[i]);
-      load_a(d, i, ko);
-    }
-#pragma unroll
-    for (int i = 0; i < W_LD; ++i) {
-      put(sa + 3 * A_PLANE, W_RUN, W_PLANE, (tid + i * NT) / QPR, rw[d][i], ow[i]);
-      load_w(d, i, ko);
+    if (c < A_LD) {
+      if (!whole) ra[d][c] = live ? ra[d][c] : u32x4_t{0, 0, 0, 0};
+      put(sa, A_RUN, A_PLANE, (tid + c * NT) / QPR, ra[d][c], oa[c]);
+      load_a(d, c, ko);
+    } else {
+      const int w = c - A_LD;
+      if (!whole) rw[d][w] = live ? rw[d][w] : u32x4_t{0, 0, 0, 0};
+      put(sa + 3 * A_PLANE, W_RUN, W_PLANE, (tid + w * NT) / QPR, rw[d][w], ow[w]);
+      load_w(d, w, ko);
     }
   };
   // A group of one wave shares its buffers with no other wave.
@@ -164,7 +159,8 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
 #pragma unroll
     for (int i = 0; i < W_LD; ++i) load_w(d, i, ko);
   }
-  put_all(0, grp, 0, grp + PD * KG, false);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) put_chunk(c, 0, grp, 0, koff(grp + PD * KG), false);
   stage_sync();
   // One step: multiply stage it (buffer it & 1) and put stage it + 1 (register
   // set d) into the other buffer.
@@ -179,13 +175,27 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
 #pragma unroll
       for (int j = 0; j < TN; ++j) wf[p][j] = *reinterpret_cast<const u32x4_t*>(sw + p * W_PLANE + j * 512);
     }
-    put_all(d, (it + 1) * KG + grp, buf ^ 1, (it + 1 + PD) * KG + grp, whole);
+    // The next stage's chunks go between the MFMAs, one MFMA and its share of
+    // the splitting at a time, so that the vector unit works while the matrix
+    // core does (16384 x 3072 x 768 450 -> 406 us, 4096 x 768 x 3072 127 -> 121,
+    // against the whole split before the first MFMA, which also spilled).
+    constexpr int NMF = 6 * TM * TN;
+    const int kt = (it + 1) * KG + grp;
+    const uint32_t ko = koff((it + 1 + PD) * KG + grp);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < 6; ++t)
+    for (int c = 0; c < NCH; ++c) {
+      put_chunk(c, d, kt, buf ^ 1, ko, whole);
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int x = c * NMF / NCH; x < (c + 1) * NMF / NCH; ++x)
+        mfma32(wf[kSplitA[x / (TM * TN)]][x % TN], af[kSplitB[x / (TM * TN)]][x / TN % TM], acc[x / TN % TM][x % TN]);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) mfma32(wf[kSplitA[t]][j], af[kSplitB[t]][i], acc[i][j]);
+      for (int x = c * NMF / NCH; x < (c + 1) * NMF / NCH; ++x) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                              // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, (32 * NCH + NMF - 1) / NMF, 0);  // VALU
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     stage_sync();
   };
   if constexpr (PD == 1) {
@@ -361,7 +371,7 @@ static int launch_split_epi(int tile, const void* a, const void* w, const void* 
 //    87 x 768 x 3072 77 -> 20 (64x64 38), 87 x 2304 x 768 23 -> 8.8; four
 //    beyond (two blocks a CU), 65 x 3072 x 768 22 -> 12.2 (eight: 15).
 static int split_tile(int M, int N, int K, bool vec_store) {
-  const int64_t cus = 256;
+  const int64_t cus = num_cus();
   auto tiles = [&](int bm, int bn) {
     return static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   };
