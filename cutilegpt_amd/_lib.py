@@ -48,6 +48,11 @@ SIGNATURES = {
                                       _I, _I, _P]),
     "cgpt_gemm_partials": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P]),
     "cgpt_gemm_partials_plan": (_I, [_I64, _I64, _I64, _I, _P]),
+    "cgpt_decode_fused_ok": (_I, [_I64, _I64, _I64, _I64, _I64, _I]),
+    "cgpt_gemm_partials_ln": (_I, [_P, _P, _I64, _I64, _I64, _P, _P, _P, _P, _F, _P, _P, _I64, _I64,
+                                   _I64, _I64, _I64, _I64, _P]),
+    "cgpt_gemm_partials_gelu": (_I, [_P, _I64, _I64, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _I64,
+                                     _I64, _P]),
     "cgpt_attention_fwd": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64,
                                 _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                                 _I64, _I64, _I64, _F, _I, _I, _P]),

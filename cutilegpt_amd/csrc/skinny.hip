@@ -605,6 +605,202 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_kernel(
 #endif  // __HIP_DEVICE_COMPILE__
 }
 
+// Decode form for one or two rows that makes its own A: the GEMM's operand is
+// the consumer pass over the previous GEMM's partial products (residual +
+// LayerNorm, or bias + GELU), which every block repeats for its K chunk instead
+// of reading a launch's result.  At so few rows the pass is a few KB a block,
+// and the launch it saves outweighs the repeats: GPT-2, one sequence, LayerNorm
+// 2.8 + GEMM 3.8 -> 4.7 us, bias + GELU 2.1 + GEMM 4.1 -> 3.9 us, a step of 24
+// tokens after 500 402 -> 335 us.
+//  * kProLn: row m = LayerNorm(x + P[0] + .. + P[n-1] + bias), over all `cols`
+//    columns in every block; block 0 stores the new residual row to x_out, a
+//    buffer other blocks do not read.
+//  * kProGelu: A[m][c] = gelu(P[0] + .. + P[n-1] + bias), for the chunk alone.
+// The arithmetic is that of add_layernorm_partials_kernel and
+// partials_bias_act_kernel (layernorm.hip, decode.hip).  K % 64 == 0.
+enum DecPro { kProLn = 0, kProGelu = 1 };
+struct DecProIn {
+  const float* parts;   // P[s] at parts + s * part_stride, rows of ldp
+  int n_parts, part_stride, ldp;
+  const bf16_t* bias;
+  const float* x;       // kProLn: residual rows of `cols`
+  float* x_out;
+  const bf16_t* gamma;
+  const bf16_t* beta;
+  float eps;
+};
+constexpr int kProMaxRows = 2;
+
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ void bf16x4_to_f32(const u32x2_t& w, float* v) {
+  v[0] = __uint_as_float(w[0] << 16);
+  v[1] = __uint_as_float(w[0] & 0xffff0000u);
+  v[2] = __uint_as_float(w[1] << 16);
+  v[3] = __uint_as_float(w[1] & 0xffff0000u);
+}
+#endif
+
+template <int PRO, int NW, int KS, int MAXP, int ROWS>
+__global__ __launch_bounds__(64 * NW) void gemm_decode_pro_kernel(
+    DecProIn in, const bf16_t* W, float* __restrict__ out, int N, int K, int ldw, int ldp, int split,
+    int chunk) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int NT = 64 * NW, KD = 64;
+  constexpr int RS = (KS * 8 + 1) * 16;  // LDS bytes per A row, one slot of padding
+  // A thread's column groups: of a row in all (K <= 2048), or of the chunk.
+  constexpr int COLS = PRO == kProLn ? 2048 : KS * KD;
+  constexpr int G = (COLS / 4 + NT - 1) / NT;
+  // Rows past ROWS are never written: their sums are dropped.
+  __shared__ __attribute__((aligned(16))) uint8_t sa[16 * RS];
+  __shared__ float scr[2][NW];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int gi = blockIdx.x / split, sk = blockIdx.x % split;
+  const int d0 = sk * chunk, d1 = min(K / KD, d0 + chunk);
+  const int c0 = d0 * KD, c1 = d1 * KD;  // the chunk's columns
+
+  // The pass's loads go out first, then the W tile's: vmcnt retires in order,
+  // so the pass waits for its own alone.
+  const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(in.parts), 0, in.n_parts * in.part_stride * 4, 0x00020000);
+  u32x4_t pv[ROWS][G][MAXP];
+  f32x4_t xv[ROWS][G];
+  u32x2_t bi[G], gm[G], bt[G];
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int c = (PRO == kProLn ? 0 : c0) + (q * NT + tid) * 4;
+    const int cc = c < (PRO == kProLn ? K : c1) ? c : 0;
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m) {
+#pragma unroll
+      for (int s = 0; s < MAXP; ++s)
+        pv[m][q][s] = s < in.n_parts ? __builtin_amdgcn_raw_buffer_load_b128(
+                                           rp, static_cast<uint32_t>((s * in.part_stride + m * in.ldp + cc) * 4), 0, 0)
+                                     : u32x4_t{0, 0, 0, 0};
+      if (PRO == kProLn) xv[m][q] = *reinterpret_cast<const f32x4_t*>(in.x + m * K + cc);
+    }
+    bi[q] = *reinterpret_cast<const u32x2_t*>(in.bias + cc);
+    if (PRO == kProLn) {
+      gm[q] = *reinterpret_cast<const u32x2_t*>(in.gamma + cc);
+      bt[q] = *reinterpret_cast<const u32x2_t*>(in.beta + cc);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t*>(W), 0, static_cast<int>((N - 1) * ldw * 2 + K * 2), 0x00020000);
+  const int nt = gi * NW + wave;
+  const bool live = nt * 16 < N;
+  const uint32_t wro = static_cast<uint32_t>(min(nt * 16 + r16, N - 1)) * ldw * 2;
+  u32x4_t wf[KS][2];
+#pragma unroll
+  for (int u = 0; u < KS; ++u)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = (d0 + u) * KD + g * 16 + h * 8;
+      wf[u][h] = __builtin_amdgcn_raw_buffer_load_b128(
+          rw, live && d0 + u < d1 ? wro + static_cast<uint32_t>(k) * 2 : kOob, 0, 0);
+    }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // Sums of the partials, in chunk order, plus the bias.
+  float v[ROWS][G][4];
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m)
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      float b[4];
+      bf16x4_to_f32(bi[q], b);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float t = __uint_as_float(pv[m][q][0][e]);
+#pragma unroll
+        for (int s = 1; s < MAXP; ++s) t += __uint_as_float(pv[m][q][s][e]);
+        v[m][q][e] = t + b[e];
+      }
+    }
+  auto put = [&](int m, int c, const float* o) {  // four columns of the chunk
+    *reinterpret_cast<u32x2_t*>(sa + m * RS + (c - c0) * 2) = u32x2_t{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+  };
+  if constexpr (PRO == kProGelu) {
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m)
+#pragma unroll
+      for (int q = 0; q < G; ++q) {
+        const int c = c0 + (q * NT + tid) * 4;
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = gelu_tanh(v[m][q][e]);
+        if (c < c1) put(m, c, o);
+      }
+  } else {
+    const float n_f = static_cast<float>(K);
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m) {
+      float sum = 0.f;
+#pragma unroll
+      for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[m][q][e] = (q * NT + tid) * 4 < K ? xv[m][q][e] + v[m][q][e] : 0.f;
+          sum += v[m][q][e];
+        }
+      auto block_sum = [&](float s, float* part) {
+        s = wave_sum(s);
+        if (lane == 0) part[wave] = s;
+        wait_lgkm0();
+        raw_barrier();
+        float t = part[0];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) t += part[w];
+        return t;
+      };
+      const float mean = block_sum(sum, scr[0]) / n_f;
+      float sq = 0.f;
+#pragma unroll
+      for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float t = v[m][q][e] - mean;
+          sq += (q * NT + tid) * 4 < K ? t * t : 0.f;
+        }
+      const float rstd = 1.0f / sqrtf(block_sum(sq, scr[1]) / n_f + in.eps);
+#pragma unroll
+      for (int q = 0; q < G; ++q) {
+        const int c = (q * NT + tid) * 4;
+        if (c < K && blockIdx.x == 0) store_vec(in.x_out + m * K + c, v[m][q]);
+        float gv[4], bv[4], o[4];
+        bf16x4_to_f32(gm[q], gv);
+        bf16x4_to_f32(bt[q], bv);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (v[m][q][e] - mean) * rstd * gv[e] + bv[e];
+        if (c >= c0 && c < c1) put(m, c, o);
+      }
+      if (m + 1 < ROWS) {  // scr is read by every wave before the next row's sums
+        wait_lgkm0();
+        raw_barrier();
+      }
+    }
+  }
+  wait_lgkm0();
+  raw_barrier();
+
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  const uint8_t* abase = sa + r16 * RS + g * 32;
+#pragma unroll
+  for (int u = 0; u < KS; ++u)
+    if (d0 + u < d1) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        Mfma<bf16_t>::run(wf[u][h], *reinterpret_cast<const u32x4_t*>(abase + (u * KD + h * 8) * 2), acc);
+    }
+  // Lane (g, r16) holds P[sk][r16][16 nt + 4 g + i].
+  const int n = nt * 16 + 4 * g;
+  if (live && r16 < ROWS && n < N)
+    *reinterpret_cast<f32x4_t*>(out + (static_cast<int64_t>(sk) * ROWS + r16) * ldp + n) = acc;
+#endif  // __HIP_DEVICE_COMPILE__
+}
+
 static int skinny_num_cus() {
   int dev = 0, n = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -988,4 +1184,117 @@ int launch_gemm_partials(bool bf16_in, const void* a, const void* w, float* part
   return CGPT_OK;
 }
 
+// Whether gemm_decode_pro_kernel takes a product: N a multiple of 4, K whole
+// double slabs (a LayerNorm row at most 2048), the decode form's own plan for
+// the split with at most five double slabs a chunk (the pass's registers), and
+// at most eight partials a row for two rows, sixteen for one.
+bool decode_pro_ok(bool ln, int M, int N, int K, int64_t ldw, int n_parts) {
+  DecodePlan dp;
+  return M >= 1 && M <= kProMaxRows && N % 4 == 0 && K % 64 == 0 && (!ln || K <= 2048) && n_parts >= 1 &&
+         n_parts <= kSkMaxSplit && decode_fits(M, N, K, K, ldw) && decode_plan(M, N, K, 0, false, 0, &dp) &&
+         dp.ks <= 5;
+}
+
+template <int PRO, int NW, int KS, int MAXP>
+static void launch_pro_rows(const DecodePlan& p, const DecProIn& in, const bf16_t* W, float* out, int M,
+                            int N, int K, int ldw, int ldp, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(p.groups * p.split)), block(64 * NW);
+  if (M == 1)
+    hipLaunchKernelGGL((gemm_decode_pro_kernel<PRO, NW, KS, MAXP, 1>), grid, block, 0, s, in, W, out, N, K,
+                       ldw, ldp, p.split, p.chunk);
+  else
+    hipLaunchKernelGGL((gemm_decode_pro_kernel<PRO, NW, KS, MAXP, 2>), grid, block, 0, s, in, W, out, N, K,
+                       ldw, ldp, p.split, p.chunk);
+}
+
+template <int PRO>
+static int launch_pro(const DecProIn& in, const void* w, float* out, int M, int N, int K, int64_t ldw,
+                      int64_t ldp, int split, hipStream_t s) {
+  DecodePlan p;
+  if (!decode_plan(M, N, K, split, false, 0, &p) || p.ks > 5) return CGPT_ESHAPE;
+  const bf16_t* W = static_cast<const bf16_t*>(w);
+  const int lw = static_cast<int>(ldw), lp = static_cast<int>(ldp);
+#define CGPT_PRO_P(NW, KS)                                                              \
+  if (in.n_parts <= 8)                                                                  \
+    launch_pro_rows<PRO, NW, KS, 8>(p, in, W, out, M, N, K, lw, lp, s);                 \
+  else                                                                                  \
+    launch_pro_rows<PRO, NW, KS, 16>(p, in, W, out, M, N, K, lw, lp, s)
+#define CGPT_PRO_KS(NW)                              \
+  switch (p.ks) {                                    \
+    case 2: CGPT_PRO_P(NW, 2); break;                \
+    case 3: CGPT_PRO_P(NW, 3); break;                \
+    default: CGPT_PRO_P(NW, 5); break;               \
+  }
+  if constexpr (PRO == kProGelu) {  // a LayerNorm row is too short for 4 waves a block
+    if (p.nw == 4) {
+      CGPT_PRO_KS(4)
+      return hip_status(hipGetLastError());
+    }
+  }
+  CGPT_PRO_KS(8)
+#undef CGPT_PRO_KS
+#undef CGPT_PRO_P
+  return hip_status(hipGetLastError());
+}
+
 }  // namespace cgpt
+
+extern "C" int cgpt_decode_fused_ok(int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t n_parts, int ln) {
+  using namespace cgpt;
+  if (M < 1 || M > kProMaxRows || N < 1 || K < 1 || N > 0x7fffffff || K > 0x7fffffff || ldw < K || n_parts < 1)
+    return 0;
+  return decode_pro_ok(ln != 0, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), ldw,
+                       static_cast<int>(n_parts < 64 ? n_parts : 64)) ? 1 : 0;
+}
+
+namespace cgpt {
+// Argument checks of the two entry points below.
+static int check_pro(bool ln, const void* parts, int64_t n_parts, int64_t part_stride, int64_t ldp_in,
+                     const void* bias, const void* w, const float* out, int64_t M, int64_t N, int64_t K,
+                     int64_t ldw, int64_t ldp, int64_t n_split) {
+  auto al = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
+  if (!parts || !bias || !w || !out) return CGPT_EINVAL;
+  if (!cgpt_decode_fused_ok(M, N, K, ldw, n_parts, ln)) return CGPT_ESHAPE;
+  if (!al(parts, 16) || !al(out, 16) || !al(w, 16) || !al(bias, 8) || ldw % 8 != 0) return CGPT_EINVAL;
+  if (part_stride % 4 != 0 || ldp_in % 4 != 0 || ldp % 4 != 0 || ldp_in < K || ldp < N ||
+      part_stride < (M - 1) * ldp_in + K || ldp > 0x7fffffff)
+    return CGPT_EINVAL;
+  if (n_parts * part_stride >= (int64_t{1} << 29)) return CGPT_ESHAPE;
+  if (n_split < 1 || n_split > kSkMaxSplit) return CGPT_EINVAL;
+  return CGPT_OK;
+}
+}  // namespace cgpt
+
+extern "C" int cgpt_gemm_partials_ln(const float* x, const float* parts_in, int64_t n_parts,
+                                     int64_t part_stride, int64_t ldp_in, const void* bias, float* x_out,
+                                     const void* gamma, const void* beta, float eps, const void* w,
+                                     float* partials, int64_t M, int64_t N, int64_t K, int64_t ldw,
+                                     int64_t ldp, int64_t n_split, void* stream) {
+  using namespace cgpt;
+  const int st = check_pro(true, parts_in, n_parts, part_stride, ldp_in, bias, w, partials, M, N, K, ldw, ldp,
+                           n_split);
+  if (st != CGPT_OK) return st;
+  if (!x || !x_out || !gamma || !beta || x == x_out || partials == parts_in) return CGPT_EINVAL;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(x_out)) & 15) return CGPT_EINVAL;
+  if ((reinterpret_cast<uintptr_t>(gamma) | reinterpret_cast<uintptr_t>(beta)) & 7) return CGPT_EINVAL;
+  const DecProIn in{parts_in, static_cast<int>(n_parts), static_cast<int>(part_stride), static_cast<int>(ldp_in),
+                    static_cast<const bf16_t*>(bias), x, x_out, static_cast<const bf16_t*>(gamma),
+                    static_cast<const bf16_t*>(beta), eps};
+  return launch_pro<kProLn>(in, w, partials, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), ldw,
+                            ldp, static_cast<int>(n_split), static_cast<hipStream_t>(stream));
+}
+
+extern "C" int cgpt_gemm_partials_gelu(const float* parts_in, int64_t n_parts, int64_t part_stride,
+                                       int64_t ldp_in, const void* bias, const void* w, float* partials,
+                                       int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldp,
+                                       int64_t n_split, void* stream) {
+  using namespace cgpt;
+  const int st = check_pro(false, parts_in, n_parts, part_stride, ldp_in, bias, w, partials, M, N, K, ldw, ldp,
+                           n_split);
+  if (st != CGPT_OK) return st;
+  if (partials == parts_in) return CGPT_EINVAL;
+  const DecProIn in{parts_in, static_cast<int>(n_parts), static_cast<int>(part_stride), static_cast<int>(ldp_in),
+                    static_cast<const bf16_t*>(bias), nullptr, nullptr, nullptr, nullptr, 0.f};
+  return launch_pro<kProGelu>(in, w, partials, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), ldw,
+                              ldp, static_cast<int>(n_split), static_cast<hipStream_t>(stream));
+}

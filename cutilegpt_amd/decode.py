@@ -19,6 +19,10 @@ and every further token costs one step over B rows:
     LM head                          cgpt_gemm (skinny, N = vocab)
     greedy token                     cgpt_argmax (also written to the history)
 
+For one or two bf16 rows the two residual + LN passes and the bias + GELU pass
+are made inside the GEMM that follows them (cgpt_gemm_partials_ln,
+cgpt_gemm_partials_gelu): five launches a layer.
+
 The split-K GEMMs leave their K chunks' sums to the kernel that reads their
 output, so a weight-streaming GEMM is one memory round trip with no
 cross-block reduction; ``partials=False`` runs the earlier sequence instead
@@ -117,6 +121,14 @@ class DecodeSession:
             self.splits[(n, k)] = ns.value
             p_max = max(p_max, ns.value * B * n)
         self.parts = torch.empty(p_max if partials else 4, dtype=torch.float32, device=dev)
+        # One or two bf16 rows: the LayerNorm and GELU passes run inside the GEMM
+        # that reads them (five launches a layer instead of eight), from one
+        # partials and residual buffer into the other.
+        ok = lambda n, k, parts, ln: bool(lib.cgpt_decode_fused_ok(B, n, k, k, self.splits[parts], ln))
+        self.fused = (partials and act is torch.bfloat16 and ok(3 * D, D, (D, 4 * D), 1) and
+                      ok(4 * D, D, (D, D), 1) and ok(D, 4 * D, (4 * D, D), 0))
+        self.parts2 = torch.empty_like(self.parts) if self.fused else None
+        self.x2 = torch.empty_like(self.x) if self.fused else None
         # One split-K workspace + counter array serves every other step GEMM
         # (they run one after another on one stream and leave the counters zero).
         ws_max, cnt_max = 0, 0
@@ -211,7 +223,51 @@ class DecodeSession:
         csb, csh, cst = self.cache.strides()
         t_max = self.cache.t_max
         scale = 1.0 / math.sqrt(hd)
-        for i in range(cfg.n_layer):
+        if self.fused:
+            # src: the partials the next launch reads; x[0]: the residual rows.
+            src, dst = pp, self.parts2.data_ptr()
+            x = [px, self.x2.data_ptr()]
+            nqkv, nproj, nfc, nmlp = (self.splits[s_] for s_ in ((3 * D, D), (D, D), (4 * D, D),
+                                                                 (D, 4 * D)))
+
+            def ln_gemm(ns_in, bias, wk, w, n, ns):
+                chk(lib.cgpt_gemm_partials_ln(x[0], src, ns_in, B * D, D, bias.data_ptr(), x[1],
+                                              W[wk + ".weight"].data_ptr(),
+                                              W[wk + ".bias"].data_ptr(), 1e-5, w.data_ptr(), dst, B,
+                                              n, D, w.stride(0), n, ns, s), "gemm_partials_ln")
+                x.reverse()
+
+            for i in range(cfg.n_layer):
+                p = f"h.{i}."
+                w = W[p + "attn.c_attn.weight"]
+                if i == 0:
+                    chk(lib.cgpt_gemm_partials(ph, w.data_ptr(), dst, B, 3 * D, D, D, w.stride(0),
+                                               3 * D, nqkv, ac, s), "gemm_partials")
+                else:
+                    ln_gemm(nmlp, W[f"h.{i - 1}.mlp.c_proj.bias"], p + "ln_1", w, 3 * D, nqkv)
+                src, dst = dst, src
+                chk(lib.cgpt_attention_decode_partials(
+                    src, nqkv, B * 3 * D, 3 * D, W[p + "attn.c_attn.bias"].data_ptr(), 0, D, 2 * D,
+                    self.cache.k[i].data_ptr(), self.cache.v[i].data_ptr(), pa, B, H, hd, t_max,
+                    self.t0, pstep, csb, csh, cst, D, hd, scale, ac, self.err.data_ptr(), s),
+                    "attention_decode_partials")
+                w = W[p + "attn.c_proj.weight"]
+                chk(lib.cgpt_gemm_partials(pa, w.data_ptr(), src, B, D, D, D, w.stride(0), D, nproj, ac,
+                                           s), "gemm_partials")
+                ln_gemm(nproj, W[p + "attn.c_proj.bias"], p + "ln_2", W[p + "mlp.c_fc.weight"], 4 * D,
+                        nfc)
+                src, dst = dst, src
+                w = W[p + "mlp.c_proj.weight"]
+                chk(lib.cgpt_gemm_partials_gelu(src, nfc, B * 4 * D, 4 * D,
+                                                W[p + "mlp.c_fc.bias"].data_ptr(), w.data_ptr(), dst, B,
+                                                D, 4 * D, w.stride(0), D, nmlp, s),
+                    "gemm_partials_gelu")
+                src, dst = dst, src
+            chk(lib.cgpt_add_layernorm_partials(
+                x[0], src, nmlp, B * D, D, W[f"h.{cfg.n_layer - 1}.mlp.c_proj.bias"].data_ptr(), None,
+                W["ln_f.weight"].data_ptr(), W["ln_f.bias"].data_ptr(), ph, B, D, 1e-5, f32, f32, ac, ac,
+                s), "add_layernorm_partials")
+        for i in range(0 if self.fused else cfg.n_layer):
             p = f"h.{i}."
             last = i + 1 == cfg.n_layer
             ln_next = "ln_f" if last else f"h.{i + 1}.ln_1"

@@ -228,6 +228,31 @@ int cgpt_gemm_partials(const void* a, const void* w, float* partials, int64_t M,
  * the most the partials consumers take. */
 int cgpt_gemm_partials_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int64_t* n_split);
 
+/* Decode steps of one or two bf16 rows: the pass over the previous GEMM's
+ * split-K partial products made by the next GEMM itself, each block for what it
+ * needs of it, in place of a launch of its own.
+ *
+ * cgpt_gemm_partials_ln: row r of A is LayerNorm(s[r]) with
+ * s[r] = x[r] + P[0][r] + ... + P[n_parts-1][r] + bias (cgpt_add_layernorm_partials'
+ * arithmetic); s is stored to x_out, which must not be x.
+ * cgpt_gemm_partials_gelu: A = gelu(P[0] + ... + P[n_parts-1] + bias)
+ * (cgpt_partials_bias_act's arithmetic).
+ *
+ * P[s] at parts_in + s * part_stride, rows of ldp_in floats, K columns; W, bias,
+ * gamma, beta bf16; x, x_out (M, K) contiguous fp32.  The n_split chunk sums are
+ * written as cgpt_gemm_partials writes them; partials must not be parts_in.
+ * cgpt_decode_fused_ok: 1 when a product is taken (ln: by the first), else 0. */
+int cgpt_decode_fused_ok(int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t n_parts, int ln);
+int cgpt_gemm_partials_ln(const float* x, const float* parts_in, int64_t n_parts, int64_t part_stride,
+                          int64_t ldp_in, const void* bias, float* x_out, const void* gamma,
+                          const void* beta, float eps, const void* w, float* partials, int64_t M,
+                          int64_t N, int64_t K, int64_t ldw, int64_t ldp, int64_t n_split,
+                          void* stream);
+int cgpt_gemm_partials_gelu(const float* parts_in, int64_t n_parts, int64_t part_stride,
+                            int64_t ldp_in, const void* bias, const void* w, float* partials,
+                            int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t ldp,
+                            int64_t n_split, void* stream);
+
 /*
  * Causal (or full) softmax attention, O = softmax(Q K^T * scale + mask) V,
  * for B batches x H heads; Q has Tq rows, K/V have Tk rows (Tk >= Tq); query i
