@@ -46,12 +46,14 @@ def _require_gpu(name: str, *tensors: Optional[torch.Tensor]) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream() would build a Stream object for its pointer.
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     """Contiguous tensor whose data pointer is 16-byte aligned."""
-    t = t.contiguous()
+    if not t.is_contiguous():
+        t = t.contiguous()
     if t.data_ptr() % 16:
         t = t.clone()
     return t
@@ -73,7 +75,7 @@ def cutile_gelu(x: torch.Tensor) -> torch.Tensor:
     lib = _lib.load()
     _lib.check(lib.cgpt_gelu(xc.data_ptr(), y.data_ptr(), xc.numel(), code, _stream()),
                "cutile_gelu")
-    return y.view(x.shape)
+    return y
 
 
 # ---------------------------------------------------------------------------
@@ -146,23 +148,25 @@ def _gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], e
     n = weight.shape[0]
     if bias is not None and bias.numel() != n:
         raise ValueError(f"{name}: bias must have {n} elements")
-    a = _aligned(x.reshape(-1, k))
-    w = weight if (weight.stride(1) == 1 and weight.stride(0) % 8 == 0
-                   and weight.data_ptr() % 16 == 0) else _aligned(weight)
+    flat = x.dim() == 2
+    a = _aligned(x if flat else x.reshape(-1, k))
+    ws0, ws1 = weight.stride()
+    if ws1 != 1 or ws0 % 8 or weight.data_ptr() % 16:
+        weight = _aligned(weight)
+        ws0 = weight.stride(0)
     m = a.shape[0]
-    out_dtype = out_dtype or x.dtype
-    if out is None:
-        out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+    fresh = out is None
+    if fresh:
+        out = a.new_empty((m, n), dtype=out_dtype or x.dtype)
     b = None if bias is None else _aligned(bias)
-    lib = _lib.load()
     in_code = _dtype_code(a, name)
     t = gemm_tile(in_code, m, n, k) if tile is None else tile
-    _lib.check(lib.cgpt_gemm(
-        a.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), out.data_ptr(),
-        m, n, k, a.stride(0), w.stride(0), out.stride(0), in_code,
-        _dtype_code(b, "bias") if b is not None else 0, _dtype_code(out, "out"), epilogue, t,
+    _lib.check(_lib.load().cgpt_gemm(
+        a.data_ptr(), weight.data_ptr(), None if b is None else b.data_ptr(), out.data_ptr(),
+        m, n, k, a.stride(0), ws0, out.stride(0), in_code,
+        0 if b is None else _dtype_code(b, "bias"), _dtype_code(out, "out"), epilogue, t,
         _stream()), name)
-    return out.view(*x.shape[:-1], n)
+    return out if flat and fresh else out.view(*x.shape[:-1], n)
 
 
 def cutile_linear(x: torch.Tensor, weight: torch.Tensor,

@@ -26,6 +26,8 @@ PyTorch fallback: without libcgpt.so the forward raises.
 
 from __future__ import annotations
 
+import ctypes
+import functools
 import math
 from typing import Dict, Optional, Tuple
 
@@ -36,6 +38,13 @@ from .config import GPTConfig
 from .tiles import gemm_tile
 
 _DT = {torch.float32: _lib.CGPT_F32, torch.bfloat16: _lib.CGPT_BF16}
+
+
+@functools.lru_cache(maxsize=None)
+def _layer_keys(i: int) -> Tuple[str, ...]:
+    """Names of layer ``i``'s parameters, in ``cgpt_forward``'s order."""
+    return tuple(f"h.{i}.{n}.{p}" for n in ("ln_1", "attn.c_attn", "attn.c_proj", "ln_2", "mlp.c_fc",
+                                            "mlp.c_proj") for p in ("weight", "bias"))
 
 
 class CutileGPT:
@@ -204,7 +213,13 @@ class CutileGPT:
                   if logits_out is None else None)
         px, ph, pq, pa, pf = (t.data_ptr() for t in (x, h, qkv, att, f))
 
-        mark = probe if probe is not None else (lambda tag, start: None)
+        scale = 1.0 / math.sqrt(hd)
+        if probe is None:
+            # The whole launch sequence in one native call.
+            self._launch_forward(lib, idx, (px, ph, pq, pa, pf), cache, logits, logits_out, s)
+            return logits_out if logits_out is not None else logits[:, :V].view(B, T, V)
+
+        mark = probe
 
         def gemm(tag, a_ptr, w, b, c_ptr, n, k, epi, out_code):
             t = gemm_tile(ac, M, n, k)
@@ -231,7 +246,6 @@ class CutileGPT:
         mark("embedding", False)
         st_qkv = (T * 3 * D, hd, 3 * D)
         st_o = (T * D, hd, D)
-        scale = 1.0 / math.sqrt(hd)
         for i in range(cfg.n_layer):
             p = f"h.{i}."
             gemm("gemm_qkv", ph, W[p + "attn.c_attn.weight"], W[p + "attn.c_attn.bias"], pq,
@@ -274,6 +288,40 @@ class CutileGPT:
                           gemm_tile(ac, M, Vp, D), s), "lm_head")
         mark("lm_head", False)
         return logits[:, :V].view(B, T, V)
+
+    def _launch_forward(self, lib, idx: torch.Tensor, bufs, cache, logits: Optional[torch.Tensor],
+                        logits_out: Optional[torch.Tensor], stream: int) -> None:
+        """``_forward``'s launches through ``cgpt_forward``, from the weights as
+        the model holds them at this call."""
+        cfg, W = self.config, self.weights
+        B, T = idx.shape
+        D, V, M = cfg.n_embd, cfg.vocab_size, B * T
+        ac = _DT[self.dtype]
+        out = logits if logits_out is None else logits_out
+        if logits_out is None:
+            head = self._head_pad
+            n_head, head_tile = head.shape[0], gemm_tile(ac, M, head.shape[0], D)
+        else:
+            head, n_head, head_tile = W["lm_head.weight"], V, _lib.TILE_AUTO
+        kv = (0,) * 7
+        if cache is not None:
+            kv = (cache.k.data_ptr(), cache.v.data_ptr(), cache.k.stride(0) * cache.k.element_size(),
+                  *cache.strides(), cache.t_max)
+        vals = [B, T, D, cfg.n_head, V, cfg.n_layer, cfg.block_size, ac, idx.data_ptr(),
+                W["wte"].data_ptr(), W["wpe"].data_ptr(), W["ln_f.weight"].data_ptr(),
+                W["ln_f.bias"].data_ptr(), *bufs, self._err.data_ptr(), head.data_ptr(), head.stride(0),
+                n_head, out.data_ptr(), out.stride(0), _DT[out.dtype], head_tile,
+                int(logits_out is not None), *kv, gemm_tile(ac, M, 3 * D, D), gemm_tile(ac, M, D, D),
+                gemm_tile(ac, M, 4 * D, D), gemm_tile(ac, M, D, 4 * D)]
+        layers = []
+        for i in range(cfg.n_layer):
+            ws = [W[k] for k in _layer_keys(i)]
+            layers += [w.data_ptr() for w in ws]
+            layers += [ws[2].stride(0), ws[4].stride(0), ws[8].stride(0), ws[10].stride(0)]
+        layers += [0, 0]  # the entry past the last layer is never dereferenced
+        _lib.check(lib.cgpt_forward((ctypes.c_int64 * len(vals))(*vals),
+                                    (ctypes.c_int64 * len(layers))(*layers),
+                                    1.0 / math.sqrt(D // cfg.n_head), 1e-5, stream), "forward")
 
     def input_errors(self) -> bool:
         """True if any forward so far saw a token id outside the vocabulary

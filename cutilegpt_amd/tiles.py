@@ -75,11 +75,15 @@ TABLE: Dict[Tuple[int, int, int, int], int] = {
     (_B, 4096, 50304, 1600): 16,  # lm head      1156
 }
 
+_TABLE_NK = frozenset(key[2:] for key in TABLE)
+
 
 def gemm_tile(dtype_code: int, m: int, n: int, k: int) -> int:
     """Tile id for a GEMM problem (table hit for M's bucket, else the library
     heuristic).  fp16 inputs run the bf16 kernels on the fp16 MFMA at the same
     rate, so they share the bf16 entries."""
+    if (n, k) not in _TABLE_NK:
+        return _lib.TILE_AUTO
     if dtype_code == _lib.CGPT_F16:
         dtype_code = _lib.CGPT_BF16
     return TABLE.get((dtype_code, m_bucket(m), n, k), _lib.TILE_AUTO)

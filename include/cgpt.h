@@ -369,6 +369,21 @@ int cgpt_attention_decode_partials(const float* qkv_partials, int64_t n_parts,
                                    int64_t o_sb, int64_t o_sh, float scale, int dtype,
                                    int* err_flag, void* stream);
 
+/* A model's prefill forward: embedding + ln_1, then for every layer QKV GEMM,
+ * (cache fill,) attention, projection with the residual, ln_2, c_fc + GELU, MLP
+ * projection with the residual and the next LayerNorm, then the LM head: the
+ * launches of the entry points above, in order, on `stream`.
+ *
+ * a: [0] B, T, D, H, V, n_layer, block_size, act dtype; [8] idx (int64, B x T),
+ * wte, wpe, ln_f weight, ln_f bias; [13] x (fp32, B T x D), h, qkv, att, f (act
+ * dtype), err flag; [19] head weight, its row stride, its rows; [22] logits,
+ * row stride, dtype, tile, last (1: only each sequence's last position);
+ * [27] k cache, v cache (0: none), bytes a layer, element strides (batch, head,
+ * time), t_max; [34] tiles of the QKV, projection, c_fc and MLP projection GEMMs.
+ * layers: 16 values each: ln_1 weight and bias, then weight and bias of c_attn and
+ * attn c_proj, of ln_2, of c_fc and mlp c_proj, and the four weights' row strides. */
+int cgpt_forward(const int64_t* a, const int64_t* layers, float scale, float eps, void* stream);
+
 /*
  * Copy T positions of keys and values ((b, h, t, d) at base + b*sb + h*sh + t*st
  * + d, e.g. strided views into a fused QKV buffer) into cache rows
