@@ -1680,13 +1680,15 @@ static int cheapest_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi,
   return best;
 }
 
+constexpr int kWideN = 16384;  // LM heads
+
 // Without the residual epilogue.  Wide N (the LM heads) with a 256x192 tile for
 // every CU: 256x256 with wave-staged non-temporal stores.  Problems no
 // pipelined kernel takes: the register-staged kernel with the largest tile that
 // still gives every CU about two blocks (128x128 for long K, 128x64 otherwise).
 static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, bool kgroup) {
   const int64_t t14 = static_cast<int64_t>((M + 255) / 256) * ((N + 191) / 192);
-  if (N >= 16384 && t14 >= num_cus() && pipe_ok(16, M, N, K, lda, ldw)) return 16;
+  if (N >= kWideN && t14 >= num_cus() && pipe_ok(16, M, N, K, lda, ldw)) return 16;
   const int pick = cheapest_tile(M, N, K, lda, ldw, epi, kgroup, true);
   if (pick >= 0) return pick;
   const TileCfg* t = kBf16Tiles;
@@ -1698,6 +1700,35 @@ static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, boo
     if (blocks >= 512) return i;
   }
   return last;
+}
+
+// The skinny kernel or a tile for M <= 64 (TILE_AUTO, no residual epilogue), from
+// both timed at M = 1 to 64 over eight products, weights rotated past the caches
+// (us, skinny -> tile):
+//  * bf16: the K-group tiles wherever they take the problem.  The skinny kernel's
+//    few waves walk K in long chains and it pads rows to its 16 or 64:
+//    64 x 768 x 3072 19.5 -> 8.1, 32 x 1600 x 6400 31.6 -> 12.7,
+//    64 x 2304 x 768 8.1 -> 5.2; one row 1 x 768 x 3072 10.3 -> 7.8,
+//    1 x 2304 x 768 5.0 -> 4.9.  Two k64 steps are the least that gives two of
+//    the groups work.  Wide N (the LM heads) is weight streaming, which the
+//    skinny kernel does at 22.9 us for 32 x 50304 x 768 (tiles 26 to 34); above
+//    32 rows its accumulators leave it too few loads in flight: 64 rows
+//    44.9 -> 28.4.
+//  * fp32: the split kernel above 32 rows (64 x 768 x 3072 36.8 -> 19.8,
+//    64 x 50304 x 768 120.9 -> 72.6), and from 17 rows unless N is wide
+//    (24 x 768 x 3072 23.2 -> 19.3, but 24 x 50304 x 768 59 -> 66) or K is
+//    short (24 x 256 x 256 4.8 -> 5.6).  Up to 16 rows the skinny kernel's plain
+//    fp32 MFMAs cost less than splitting the weights: 16 x 2304 x 768 8.0 against 9.0.
+static bool skinny_bf16(int64_t M, int64_t N, int64_t K, bool wide_tile, bool kgroup) {
+  if (M > 64) return false;
+  if (N >= kWideN) return M <= 32 || !wide_tile;
+  return !kgroup || K < 128;
+}
+
+static bool skinny_f32(int64_t M, int64_t N, int64_t K, bool far) {
+  if (M > 64) return false;
+  if (far || K < 256) return true;
+  return M <= (N < kWideN && K >= 512 ? 16 : 32);
 }
 
 // Residual epilogue (C += A W^T + bias).  `tile`: 14 = the slab kernel's
@@ -1978,7 +2009,11 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
   }
   if (tile != CGPT_TILE_AUTO && tile != CGPT_TILE_SKINNY && (tile < 0 || tile >= nt))
     return CGPT_EINVAL;
-  if (tile == CGPT_TILE_AUTO && M <= 64 && !el && !f16) tile = CGPT_TILE_SKINNY;
+  if (tile == CGPT_TILE_AUTO && !el && !f16 &&
+      (bf16 ? skinny_bf16(M, N, K, pipe_ok(16, M, N, K, lda, ldw),
+                          gemm_kgroup_ok(M, N, K, lda, ldw, ldc, c, out16))
+            : skinny_f32(M, N, K, f32_far)))
+    tile = CGPT_TILE_SKINNY;
   if (tile == CGPT_TILE_SKINNY) {
     if (M > 64) return CGPT_ESHAPE;
     return launch_gemm_skinny(bf16, epilogue, a, w, bias, bb, c, out16, m, n, k, lda, ldw, ldc,

@@ -9,7 +9,9 @@
 // 2^-26 of the product, a quarter of fp32's own rounding of it, and one MFMA
 // adds 16 products at a time where the fp32 one adds 4: the error against
 // float64 is below the fp32 MFMA's (K = 768: 4.3e-7 against 5.0e-7 of the
-// result's norm, K = 6400: 1.27e-6 against 1.43e-6).
+// result's norm, K = 6400: 1.27e-6 against 1.43e-6).  The small tiles, which add
+// the small terms up apart, leave a third of that: 50 rows through a 768-wide
+// MLP 1.7e-7 (the skinny kernel 4.1e-7), 48 x 50257 x 768 8.8e-8 (1.8e-7).
 //
 // Two kinds of input cannot be represented like this, and a block that meets
 // one computes its tile again with the fp32 MFMA straight from global memory:
@@ -54,6 +56,10 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
   constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int TM = WM / 32, TN = WN / 32;
   static_assert(WM % 32 == 0 && WN % 32 == 0, "32x32 MFMA tiles");
+  // Waves of one 32x32 product have the registers to keep the five smaller
+  // products' sums (2^-8 of h h) apart: one rounding of the large sum a stage,
+  // not six, and two chains of MFMAs, not one.
+  constexpr bool kLow = TM * TN == 1;
   constexpr int BK = 16, QPR = BK / 4;  // 16-byte fp32 chunks a row and stage
   constexpr int A_LD = BM * QPR / NT, W_LD = BN * QPR / NT;
   static_assert(BM * QPR % NT == 0 && BN * QPR % NT == 0, "tile/thread mismatch");
@@ -148,6 +154,9 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  f32x16_t low;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) low[r] = 0.f;
 
   const int KT = (K + BK - 1) / BK;
   const int iters = (KT + KG - 1) / KG;  // the same for every group: a stage past K is zero
@@ -188,7 +197,8 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
       put_chunk(c, d, kt, buf ^ 1, ko, whole);
 #pragma unroll
       for (int x = c * NMF / NCH; x < (c + 1) * NMF / NCH; ++x)
-        mfma32(wf[kSplitA[x / (TM * TN)]][x % TN], af[kSplitB[x / (TM * TN)]][x / TN % TM], acc[x / TN % TM][x % TN]);
+        mfma32(wf[kSplitA[x / (TM * TN)]][x % TN], af[kSplitB[x / (TM * TN)]][x / TN % TM],
+               kLow && x > 0 ? low : acc[x / TN % TM][x % TN]);
 #pragma unroll
       for (int x = c * NMF / NCH; x < (c + 1) * NMF / NCH; ++x) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                              // MFMA
@@ -212,6 +222,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
 #pragma unroll
       for (int u = 0; u < PD; ++u) step(it + u, u & 1, (u + 1) % PD, false);
   }
+  if constexpr (kLow) acc[0][0] += low;
   if constexpr (NW == 1 && KG > 1) __syncthreads();
 
   // Each group adds the others' sums of its quads (in group order).
@@ -369,12 +380,15 @@ static int launch_split_epi(int tile, const void* a, const void* w, const void* 
 //    24 -> 15 (128x64 21, 32x32 18);
 //  * 32x32, a wave a K group: eight groups while that is one round of blocks,
 //    87 x 768 x 3072 77 -> 20 (64x64 38), 87 x 2304 x 768 23 -> 8.8; four
-//    beyond (two blocks a CU), 65 x 3072 x 768 22 -> 12.2 (eight: 15).
+//    beyond (two blocks a CU), 65 x 3072 x 768 22 -> 12.2 (eight: 15); of
+//    64 rows or fewer those beyond are one row of tiles, 64 x 4800 x 1600 26.9
+//    with 64x64 (32x32 29.2), 64 x 50304 x 768 73 (32x32 90, 128x128 78).
 static int split_tile(int M, int N, int K, bool vec_store) {
   const int64_t cus = num_cus();
   auto tiles = [&](int bm, int bn) {
     return static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   };
+  if (M <= 64) return tiles(32, 32) <= cus ? k32x32k8 : M <= 32 ? k32x32k4 : k64x64k4;
   const int64_t t256 = tiles(256, 256), rounds = (t256 + cus - 1) / cus;
   if (t256 >= cus && vec_store && 4 * t256 >= 3 * rounds * cus) return k256x256;
   const int64_t t128 = tiles(128, 128);

@@ -16,7 +16,7 @@ and every further token costs one step over B rows:
                bias + GELU           cgpt_partials_bias_act (adds the partials)
                MLP proj GEMM         cgpt_gemm_partials
                residual + next LN    cgpt_add_layernorm_partials (LN_f last)
-    LM head                          cgpt_gemm (skinny, N = vocab)
+    LM head                          cgpt_gemm (N = vocab)
     greedy token                     cgpt_argmax (also written to the history)
 
 For one or two bf16 rows the two residual + LN passes and the bias + GELU pass
@@ -186,13 +186,10 @@ class DecodeSession:
         pws, pcnt, nws, ncnt = (self.ws.data_ptr(), self.counters.data_ptr(), self.ws_bytes,
                                 self.counters.numel())
 
-        def gemm(a_ptr, w, b, c_ptr, n, k, epi, out_code, split=True):
-            # split=False: the unsplit kernel, whose wider blocks suit the wide
-            # GEMMs (c_fc, the LM head) better than the cross-block fix-up.
+        def gemm(a_ptr, w, b, c_ptr, n, k, epi, out_code):
             chk(lib.cgpt_gemm_skinny(a_ptr, w.data_ptr(), None if b is None else b.data_ptr(),
                                      c_ptr, B, n, k, k, w.stride(0), n, ac, ac, out_code, epi,
-                                     pws if split else None, nws, pcnt if split else None, ncnt,
-                                     s), "gemm_skinny")
+                                     pws, nws, pcnt, ncnt, s), "gemm_skinny")
 
         def add_ln(delta_ptr, wk, keep_x=True):
             chk(lib.cgpt_add_layernorm(px, delta_ptr, px if delta_ptr and keep_x else None,
@@ -305,8 +302,12 @@ class DecodeSession:
             gemm(pf, W[p + "mlp.c_proj.weight"], W[p + "mlp.c_proj.bias"], pd, D, 4 * D,
                  _lib.EPI_BIAS, f32)
             add_ln(pd, ln_next, keep_x=not last)
-        gemm(ph, W["lm_head.weight"], None, self.logits.data_ptr(), V, D, _lib.EPI_NONE,
-             _DT[self.logits.dtype], split=not self.partials)
+        w, code = W["lm_head.weight"], _DT[self.logits.dtype]
+        if self.partials:
+            chk(lib.cgpt_gemm(ph, w.data_ptr(), None, self.logits.data_ptr(), B, V, D, D, w.stride(0), V,
+                              ac, ac, code, _lib.EPI_NONE, _lib.TILE_AUTO, s), "gemm")
+        else:
+            gemm(ph, w, None, self.logits.data_ptr(), V, D, _lib.EPI_NONE, code)
 
     def greedy_step(self) -> None:
         """``step_logits`` + argmax into ``ids`` and history column step + 1,

@@ -139,8 +139,9 @@ int cgpt_partials_bias_act(const float* partials, int64_t n_parts, int64_t part_
  * others run a 64x64 register-staged kernel that loads element by element
  * (any tile id but CGPT_TILE_SKINNY is then ignored).  fp16 inputs run every
  * tile id as bf16 does, on the fp16 MFMA.
- * `tile` selects a tile configuration: CGPT_TILE_AUTO = library heuristic (the
- * skinny kernel when M <= 64, fp32 / bf16); CGPT_TILE_SKINNY = the
+ * `tile` selects a tile configuration: CGPT_TILE_AUTO = library heuristic (a
+ * tile, or for M <= 64 in fp32 / bf16 the skinny kernel where that is the faster
+ * one: few rows of fp32, a wide N, a K the tiles do not take); CGPT_TILE_SKINNY = the
  * weight-streaming kernel for M <= 64 rows (decode steps: one row per
  * sequence), CGPT_ESHAPE above; fp32 and bf16 under the vector rules only.
  * With CGPT_EPI_BIAS_RESID (C += A W^T + bias in place, C usually the fp32

@@ -25,6 +25,8 @@ SHAPES = [
     (2900, 772, 704), (3300, 768, 3072),                              # 128x96
     (2048, 1600, 6400), (4001, 772, 1088),                            # 128x128
     (6000, 768, 3072),                                                # 192x96
+    (1, 36, 128), (17, 100, 192), (33, 772, 1088), (64, 4800, 1600),  # 64 rows or fewer,
+    (64, 36, 64), (32, 16388, 128), (33, 16388, 128),                 # with the skinny kernel's side
 ]
 
 

@@ -50,6 +50,8 @@ SHAPES = [
     (513, 3100, 100), (520, 3072, 768),                                # 128x64, 2 groups
     (1409, 1537, 1540), (1500, 1600, 1600),                            # 128x128, 2 groups
     (2049, 5121, 44), (87, 50257, 64),                                 # 128x128
+    (16, 130, 512), (17, 130, 512), (17, 130, 508), (33, 130, 252),    # 64 rows or fewer: the skinny
+    (33, 131, 256), (64, 4800, 1600), (32, 16384, 512), (33, 16385, 512),  # kernel or a split tile
     (4095, 4100, 28), (4096, 6144, 80),                                # 256x256
 ]
 
