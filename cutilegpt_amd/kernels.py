@@ -148,7 +148,7 @@ def _gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], e
     n = weight.shape[0]
     if bias is not None and bias.numel() != n:
         raise ValueError(f"{name}: bias must have {n} elements")
-    flat = x.dim() == 2
+    flat = x.dim() == 2 and k > 0
     a = _aligned(x if flat else x.reshape(-1, k))
     ws0, ws1 = weight.stride()
     if ws1 != 1 or ws0 % 8 or weight.data_ptr() % 16:
@@ -163,7 +163,7 @@ def _gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], e
     t = gemm_tile(in_code, m, n, k) if tile is None else tile
     _lib.check(_lib.load().cgpt_gemm(
         a.data_ptr(), weight.data_ptr(), None if b is None else b.data_ptr(), out.data_ptr(),
-        m, n, k, a.stride(0), ws0, out.stride(0), in_code,
+        m, n, k, k, ws0, out.stride(0), in_code,  # (a one-row view may have any row stride)
         0 if b is None else _dtype_code(b, "bias"), _dtype_code(out, "out"), epilogue, t,
         _stream()), name)
     return out if flat and fresh else out.view(*x.shape[:-1], n)

@@ -76,3 +76,21 @@ def test_kgroup_repeats_bit_for_bit(gpu):
     a, w, b, _ = problem(gpu, 97, 768, 3072, BF16)
     outs = [gemm(gpu, a, w, b, _lib.EPI_BIAS, torch.empty(97, 768, device=gpu)) for _ in range(3)]
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16, F32])
+@pytest.mark.parametrize("row,width", [(0, 772), (2, 772), (0, 769), (1, 769)])
+def test_one_row_view(gpu, row, width, dtype):
+    """A one-row view counts as contiguous whatever its row stride: neither that
+    stride nor its alignment reaches the kernels."""
+    from cutilegpt_amd.kernels import cutile_linear_bias
+
+    a, w, b, ref = problem(gpu, 3, 100, 768, dtype)
+    wide = torch.zeros(3, width, dtype=dtype, device=gpu)
+    wide[:, :768] = a
+    out = cutile_linear_bias(wide[row:row + 1, :768], w, b)
+    # bit for bit the same kernel's result as for rows of their own
+    assert torch.equal(out, cutile_linear_bias(a[row:row + 1].clone(), w, b))
+    # 16 bits: one rounding of the output; fp32: sqrt(768) roundings of the running sum
+    tol = {F32: 2.0 ** -18, F16: 2.0 ** -10, BF16: 2.0 ** -7}[dtype]
+    assert (out.double() - ref[row:row + 1]).abs().max() <= tol * ref.abs().max()
