@@ -1661,7 +1661,8 @@ static float tile_cost(const TileCost& t, uint32_t M, uint32_t N, float k64, flo
 // The cheapest tile that takes the problem; -1 when none does (K % 64 != 0, or
 // operands past the pipelines' 32-bit offsets).  kgroup, slab: whether
 // gemm_kgroup.hip's tiles and (residual epilogue) the slab kernel take it.
-static int cheapest_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, bool kgroup, bool slab) {
+static int cheapest_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, bool kgroup, bool slab,
+                         float* us_out = nullptr) {
   const bool resid = epi == CGPT_EPI_BIAS_RESID;
   const uint32_t cus = num_cus(), m = M, n = N;
   const float k64 = static_cast<float>(K) / 64, mn = static_cast<float>(M) * static_cast<float>(N) * 1e-6f;
@@ -1677,7 +1678,38 @@ static int cheapest_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi,
       best_us = us;
     }
   }
+  if (us_out != nullptr) *us_out = best_us;
   return best;
+}
+
+// Wide N in 256x256 tiles: the columns of the tiles that fill whole rounds of
+// the CUs when the last ones are better left to a second launch of smaller
+// tiles; 0: one launch.  A last round of a few tiles keeps the other CUs idle
+// for as long as a full one: 1000 x 50257 x 768 (bf16 out) is 788 tiles, three
+// rounds and 20 tiles, 116.4 -> 102.9 us in two launches; 1000 x 50304 x 1600
+// (fp32 out) 186.4 -> 164.0, 300 x 50257 x 1600 101.1 -> 88.0, 3000 x 50304 x
+// 1600 499 -> 479.  The CUs drift apart over many rounds and share the last one
+// better than predicted: heads with less than 2.5% to gain ran 0.97 to 1.03
+// times as fast (4096 x 50304 x 768, 0.8% predicted, 342 -> 352), those above
+// it 1.01 to 1.18.  Narrower products gained and lost (0.94 to 1.07).
+static int64_t whole_round_columns(int tile, int M, int N, int K, int64_t lda, int64_t ldw, int epi,
+                                   bool kgroup) {
+  const TileCost* t = kTileCosts;
+  while (t->id != tile) ++t;
+  const int64_t cus = num_cus(), tiles_m = (M + t->bm - 1) / t->bm, tiles_n = (N + t->bn - 1) / t->bn;
+  const int64_t cols = tiles_m * tiles_n / cus * cus / tiles_m;  // column tiles of the full rounds
+  if (cols == 0 || cols >= tiles_n) return 0;
+  const int n1 = static_cast<int>(cols * t->bn), rest = N - n1;
+  const float k64 = static_cast<float>(K) / 64, k_mb = static_cast<float>(K) * 2e-6f;
+  const float m = static_cast<float>(M);
+  auto cost = [&](int n) {
+    const float nf = static_cast<float>(n);
+    return tile_cost(*t, M, n, k64, m * nf * 1e-6f, (m + nf) * k_mb, epi, static_cast<uint32_t>(cus));
+  };
+  float rest_us = 0.f;
+  if (cheapest_tile(M, rest, K, lda, ldw, epi, kgroup, true, &rest_us) < 0) return 0;
+  constexpr float kLaunchUs = 2.f;  // the second launch
+  return cost(n1) + rest_us + kLaunchUs < 0.975f * cost(N) ? n1 : 0;
 }
 
 constexpr int kWideN = 16384;  // LM heads
@@ -2022,7 +2054,20 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
   el = el || f32_far;
   if (el) tile = 0;  // the element-load kernel has one tile
   if (tile == CGPT_TILE_AUTO && (bf16 || f16)) {
-    tile = auto_tile(m, n, k, lda, ldw, epilogue, gemm_kgroup_ok(M, N, K, lda, ldw, ldc, c, out16));
+    const bool kgroup = gemm_kgroup_ok(M, N, K, lda, ldw, ldc, c, out16);
+    tile = auto_tile(m, n, k, lda, ldw, epilogue, kgroup);
+    const int64_t n1 =
+        tile == 16 && N >= kWideN ? whole_round_columns(tile, m, n, k, lda, ldw, epilogue, kgroup) : 0;
+    if (n1 > 0) {
+      const int rc = cgpt_gemm(a, w, bias, c, M, n1, K, lda, ldw, ldc, in_dtype, bias_dtype, out_dtype,
+                               epilogue, tile, stream);
+      if (rc != CGPT_OK) return rc;
+      const uint8_t* b = static_cast<const uint8_t*>(bias);
+      return cgpt_gemm(a, static_cast<const uint8_t*>(w) + n1 * ldw * 2,
+                       b == nullptr ? nullptr : b + n1 * (bb ? 2 : 4),
+                       static_cast<uint8_t*>(c) + n1 * (out16 ? 2 : 4), M, N - n1, K, lda, ldw, ldc, in_dtype,
+                       bias_dtype, out_dtype, epilogue, CGPT_TILE_AUTO, stream);
+    }
     if (tile >= kFirstKgroupTile)
       return launch_gemm_kgroup(f16, epilogue, tile - kFirstKgroupTile, a, w, bias, bb, c, out16, m, n, k,
                                 lda, ldw, ldc, s);

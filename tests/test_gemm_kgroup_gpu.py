@@ -78,6 +78,30 @@ def test_kgroup_repeats_bit_for_bit(gpu):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("epi", [_lib.EPI_NONE, _lib.EPI_BIAS, _lib.EPI_BIAS_GELU])
+@pytest.mark.parametrize("out_dtype", [BF16, F32])
+@pytest.mark.parametrize("m,n,k,pad", [
+    (1000, 16388, 128, 0), (1000, 16388, 128, 3),  # one round of 256x256 tiles and 4 columns
+    (1000, 16391, 128, 0),                         # ... and 7, rows of odd length
+    (300, 33000, 192, 8),                          # two tile rows, 232 columns left
+    (1000, 16384, 128, 0),                         # whole rounds: one launch
+])
+def test_wide_n_whole_rounds(gpu, m, n, k, pad, out_dtype, epi):
+    """Wide N whose last columns go to a second launch: both parts, and nothing
+    past them."""
+    a, w, b, ref = problem(gpu, m, n, k, BF16)
+    if epi == _lib.EPI_NONE:
+        ref = ref - b.double()
+    elif epi == _lib.EPI_BIAS_GELU:
+        ref = torch.nn.functional.gelu(ref, approximate="tanh")
+    out = torch.full((m, n + pad), 7.0, dtype=out_dtype, device=gpu)
+    gemm(gpu, a, w, b, epi, out[:, :n], F32 if pad else None)
+    # as above; a bf16 output adds its rounding
+    tol = 1e-4 * math.sqrt(k / 64) + (1e-5 if out_dtype is F32 else 2.0 ** -8) * ref.abs().max()
+    assert (out[:, :n].double() - ref).abs().max() <= tol
+    assert (out[:, n:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16, F32])
 @pytest.mark.parametrize("row,width", [(0, 772), (2, 772), (0, 769), (1, 769)])
 def test_one_row_view(gpu, row, width, dtype):
