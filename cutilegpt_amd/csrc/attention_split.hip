@@ -193,7 +193,8 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
   };
 
   for (int j = 0; j < n_kv; ++j) {
-    raw_barrier();  // every wave is done reading the previous block
+    wait_lgkm0();
+    raw_barrier();  // every wave's reads of the previous block have landed
     swrite();
     if (j + 1 < n_kv) gload(j + 1);
     wait_lgkm0();
