@@ -137,11 +137,11 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
       const int row = lrow + i * (kAsThreads / CPR);
       const int at = row * KROW + (((lchunk >> 1) ^ (row & 7)) << 4) + (lchunk & 1) * 8;
       u32x2_t hh, mm, ll;
-      split3(rk[i], hh, mm, ll);
+      split3(rk[i], 1.0f, hh, mm, ll);
       *reinterpret_cast<u32x2_t*>(sk + at) = hh;
       *reinterpret_cast<u32x2_t*>(sk + PLANE + at) = mm;
       *reinterpret_cast<u32x2_t*>(sk + 2 * PLANE + at) = ll;
-      split3(rv[i], hh, mm, ll);
+      split3(rv[i], 1.0f, hh, mm, ll);
       *reinterpret_cast<u32x2_t*>(sv + at) = hh;
       *reinterpret_cast<u32x2_t*>(sv + PLANE + at) = mm;
       *reinterpret_cast<u32x2_t*>(sv + 2 * PLANE + at) = ll;
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
         u32x4_t v = *reinterpret_cast<const u32x4_t*>(p + 4 * x);
         if (qi >= Tq) v = u32x4_t{0, 0, 0, 0};
         u32x2_t hh, mm, ll;
-        split3(v, hh, mm, ll);
+        split3(v, 1.0f, hh, mm, ll);
         qf[0][qt][ks][2 * x] = hh[0], qf[0][qt][ks][2 * x + 1] = hh[1];
         qf[1][qt][ks][2 * x] = mm[0], qf[1][qt][ks][2 * x + 1] = mm[1];
         qf[2][qt][ks][2 * x] = ll[0], qf[2][qt][ks][2 * x + 1] = ll[1];
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
           u32x2_t hh, mm, ll;
-          split3(__builtin_bit_cast(u32x4_t, s[qt][2 * c + x]), hh, mm, ll);
+          split3(__builtin_bit_cast(u32x4_t, s[qt][2 * c + x]), 1.0f, hh, mm, ll);
           pf[0][qt][2 * x] = hh[0], pf[0][qt][2 * x + 1] = hh[1];
           pf[1][qt][2 * x] = mm[0], pf[1][qt][2 * x + 1] = mm[1];
           pf[2][qt][2 * x] = ll[0], pf[2][qt][2 * x + 1] = ll[1];
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
   bool odd = chk != chk;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    odd = odd || ((seen[e] & 0x7fffffffu) != 0 && (seen[e] & kSplitNormalBits) == 0);
+    odd = odd || ((seen[e] & 0x7fffffffu) != 0 && (seen[e] & 0x70000000u) == 0);
   const bool redo = __syncthreads_or(odd) != 0;
   if (!wave_live) return;
 #pragma unroll

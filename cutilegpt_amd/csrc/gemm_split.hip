@@ -13,13 +13,11 @@
 // the small terms up apart, leave a third of that: 50 rows through a 768-wide
 // MLP 1.7e-7 (the skinny kernel 4.1e-7), 48 x 50257 x 768 8.8e-8 (1.8e-7).
 //
-// Two kinds of input cannot be represented like this, and a block that meets
-// one computes its tile again with the fp32 MFMA straight from global memory:
-//  * infinities, NaN and sums that overflow: the parts of an infinity (or of a
-//    value that rounds to one in bf16) are infinite or NaN, and so is every
-//    sum they enter, so accumulators that are not all finite tell;
-//  * rows of A or W whose values are all below 2^-95: their l parts run into
-//    bf16's subnormals.  The loader ORs the exponent bits of every row chunk.
+// Both operands are split at 2^23 times their size (split.h), so that no part of
+// a small value is subnormal, and the sums are scaled back by 2^-46.  A block
+// whose sums are not all finite computes its tile again with the fp32 MFMA
+// straight from global memory: infinities, NaN, values of 2^105 and more, and
+// sums of 2^82 and more (those that overflow fp32 among them).
 #include "common.h"
 #include "gemm_common.h"
 #include "internal.h"
@@ -99,11 +97,6 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
     wo[i] = static_cast<uint32_t>(min((tid + i * NT) / QPR, N - 1 - n0) * ldw) * 4;
   const int kq = tid % QPR;
   u32x4_t ra[PD][A_LD], rw[PD][W_LD];
-  uint32_t oa[A_LD], ow[W_LD];  // OR of the values seen, by row
-#pragma unroll
-  for (int i = 0; i < A_LD; ++i) oa[i] = 0;
-#pragma unroll
-  for (int i = 0; i < W_LD; ++i) ow[i] = 0;
   // k past K is loaded from the row's last chunk and zeroed before the split.
   auto koff = [&](int kt) { return static_cast<uint32_t>(min(kt * BK + kq * 4, K - 4)) * 4; };
   auto load_a = [&](int d, int i, uint32_t ko) {
@@ -112,11 +105,9 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
   auto load_w = [&](int d, int i, uint32_t ko) {
     rw[d][i] = *reinterpret_cast<const u32x4_t*>(wb + (wo[i] + ko));
   };
-  auto put = [&](uint8_t* base, int run, int plane, int row, const u32x4_t& v, uint32_t& seen) {
+  auto put = [&](uint8_t* base, int run, int plane, int row, const u32x4_t& v) {
     u32x2_t h, m, l;
-    split3(v, h, m, l);
-    seen = v[0] | v[1] | seen;
-    seen = v[2] | v[3] | seen;
+    split3(v, kSplitUp, h, m, l);
     uint8_t* p = base + (kq >> 1) * run + row * 16 + (kq & 1) * 8;
     *reinterpret_cast<u32x2_t*>(p) = h;
     *reinterpret_cast<u32x2_t*>(p + plane) = m;
@@ -132,12 +123,12 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
     uint8_t* sa = gbase + buf * STAGE;
     if (c < A_LD) {
       if (!whole) ra[d][c] = live ? ra[d][c] : u32x4_t{0, 0, 0, 0};
-      put(sa, A_RUN, A_PLANE, (tid + c * NT) / QPR, ra[d][c], oa[c]);
+      put(sa, A_RUN, A_PLANE, (tid + c * NT) / QPR, ra[d][c]);
       load_a(d, c, ko);
     } else {
       const int w = c - A_LD;
       if (!whole) rw[d][w] = live ? rw[d][w] : u32x4_t{0, 0, 0, 0};
-      put(sa + 3 * A_PLANE, W_RUN, W_PLANE, (tid + w * NT) / QPR, rw[d][w], ow[w]);
+      put(sa + 3 * A_PLANE, W_RUN, W_PLANE, (tid + w * NT) / QPR, rw[d][w]);
       load_w(d, w, ko);
     }
   };
@@ -256,18 +247,6 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
     }
   }
 
-  // A row of A or W (this group's share of its k) that is not zero and has no
-  // value of 2^-95 or above.
-  bool tiny = false;
-  auto check_row = [&](uint32_t v) {
-    v |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kDppXor1, 0xF, 0xF, true));
-    v |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kDppXor2, 0xF, 0xF, true));
-    tiny = tiny || ((v & 0x7fffffffu) != 0 && (v & kSplitNormalBits) == 0);
-  };
-#pragma unroll
-  for (int i = 0; i < A_LD; ++i) check_row(oa[i]);
-#pragma unroll
-  for (int i = 0; i < W_LD; ++i) check_row(ow[i]);
   // x * 0 is NaN exactly for infinities and NaN.
   float chk = 0.f;
 #pragma unroll
@@ -276,7 +255,9 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         chk = __builtin_fmaf(acc[q / 4 / TN][q / 4 % TN][4 * (q % 4) + r], 0.f, chk);
-  if (__syncthreads_or(tiny || chk != chk)) {
+  float down = kSplitDown * kSplitDown;
+  if (__syncthreads_or(chk != chk)) {
+    down = 1.0f;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -305,7 +286,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
     float v[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float t = acc[i][j][e + r];
+      float t = acc[i][j][e + r] * down;
       if (EPI != CGPT_EPI_NONE && n + r < N)
         t += bias_bf16 ? bf16_to_f32(static_cast<const bf16_t*>(bias)[n + r])
                        : static_cast<const float*>(bias)[n + r];

@@ -117,3 +117,34 @@ def test_split_tiny_rows(gpu, scale):
     row = (out.double() - ref).norm(dim=1) / ref.norm(dim=1)
     # Products of subnormal results carry absolute errors of 2^-149 each.
     assert row.max() < 4 * 2.0 ** -24 * math.sqrt(k), row.max()
+
+
+# Small elements in rows that hold ordinary ones too, each against a partner of
+# the inverse scale; e < 0: in W.  Products are of order one, so the bound of
+# `check` holds with the sum of their sizes for the norms.
+@pytest.mark.parametrize("e", [-125, -115, -100, -80, 80, 100, 106, 115, 125])
+@pytest.mark.parametrize("m,n,k", [(97, 31, 64), (300, 1000, 36), (200, 3000, 52), (513, 3100, 100),
+                                   (1409, 1537, 1540), (2049, 5121, 32), (4095, 4100, 28)])
+def test_split_inverse_scales(gpu, m, n, k, e):
+    a, w = randn(gpu, m, k, seed=1), randn(gpu, n, k, seed=2)
+    a[:, 1::2] *= 2.0 ** -e
+    w[:, 1::2] *= 2.0 ** e
+    w[:, 0] = 0.0                    # nothing large against the ordinary a[:, 0]
+    ref = a.double() @ w.double().t()
+    size = a.double().abs() @ w.double().abs().t()
+    out = run(gpu, a, w, None, _lib.EPI_NONE)
+    tol = 4 * 2.0 ** -24 * math.sqrt(6 * k / 16 + 16)
+    assert ((out.double() - ref).abs() / size).max() <= tol
+
+
+@pytest.mark.parametrize("scale", [1e-38, 1e-42, 1e-44])
+def test_split_smallest_values(gpu, scale):
+    """Small and subnormal values beside ordinary ones that meet zeros."""
+    m, n, k = 100, 90, 64
+    a, w = randn(gpu, m, k, seed=1), randn(gpu, n, k, seed=2) * 1e30
+    a[:, ::2] *= scale
+    w[:, 1::2] = 0.0
+    ref = a.double() @ w.double().t()
+    size = a.double().abs() @ w.double().abs().t()
+    out = run(gpu, a, w, None, _lib.EPI_NONE)
+    assert ((out.double() - ref).abs() / size).max() <= 4 * 2.0 ** -24 * math.sqrt(k)
