@@ -11,10 +11,12 @@
 // plane, the planes of one key block filling 48 KiB (three blocks a CU hide the
 // two barriers around a refill).
 //
-// A block whose sums are not all finite (infinities or NaN in the inputs,
-// values that round to infinity in bf16) or that met a column of V with values
-// all below 2^-95, whose parts bf16 cannot hold, computes its rows again with
-// the fp32 MFMA.  (Q and K that small change no score by more than 2^-100.)
+// K, V and P are split at 2^23 times their size (split.h: no part of a small
+// value is subnormal), Q at 2^-23, so that the scores keep their size and
+// overflow where fp32's do; the sums of P V are scaled back with the normaliser.
+// A block whose sums are not all finite (infinities or NaN in the inputs, values
+// of K and V of 2^105 and more) or whose Q has a value below 2^-80, whose scaled
+// parts bf16 cannot hold, computes its rows again with the fp32 MFMA.
 #include "common.h"
 #include "internal.h"
 #include "split.h"
@@ -121,7 +123,6 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
   // Thread (row tid / CPR, chunk tid % CPR) of every 16 rows.
   const int lrow = tid / CPR, lchunk = tid % CPR;
   u32x4_t rk[LD], rv[LD];
-  u32x4_t seen = {0, 0, 0, 0};  // OR of the V values of each of the chunk's columns
   auto gload = [&](int j) {
 #pragma unroll
     for (int i = 0; i < LD; ++i) {
@@ -137,21 +138,21 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
       const int row = lrow + i * (kAsThreads / CPR);
       const int at = row * KROW + (((lchunk >> 1) ^ (row & 7)) << 4) + (lchunk & 1) * 8;
       u32x2_t hh, mm, ll;
-      split3(rk[i], 1.0f, hh, mm, ll);
+      split3(rk[i], kSplitUp, hh, mm, ll);
       *reinterpret_cast<u32x2_t*>(sk + at) = hh;
       *reinterpret_cast<u32x2_t*>(sk + PLANE + at) = mm;
       *reinterpret_cast<u32x2_t*>(sk + 2 * PLANE + at) = ll;
-      split3(rv[i], 1.0f, hh, mm, ll);
+      split3(rv[i], kSplitUp, hh, mm, ll);
       *reinterpret_cast<u32x2_t*>(sv + at) = hh;
       *reinterpret_cast<u32x2_t*>(sv + PLANE + at) = mm;
       *reinterpret_cast<u32x2_t*>(sv + 2 * PLANE + at) = ll;
-      seen |= rv[i];
     }
   };
 
   gload(0);
   // Q's parts stay in registers for the whole key loop (rows past Tq: zero).
   u32x4_t qf[3][QT][NKS];
+  bool odd = false;  // what the split does not hold was met
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     const int qi = q0 + wave * 16 * QT + qt * 16 + frow;
@@ -162,8 +163,10 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
       for (int x = 0; x < 2; ++x) {
         u32x4_t v = *reinterpret_cast<const u32x4_t*>(p + 4 * x);
         if (qi >= Tq) v = u32x4_t{0, 0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) odd = odd || (v[e] << 1) - 1 < ((127u - 80) << 24) - 1;  // 0 < |v| < 2^-80
         u32x2_t hh, mm, ll;
-        split3(v, 1.0f, hh, mm, ll);
+        split3(v, kSplitDown, hh, mm, ll);
         qf[0][qt][ks][2 * x] = hh[0], qf[0][qt][ks][2 * x + 1] = hh[1];
         qf[1][qt][ks][2 * x] = mm[0], qf[1][qt][ks][2 * x + 1] = mm[1];
         qf[2][qt][ks][2 * x] = ll[0], qf[2][qt][ks][2 * x + 1] = ll[1];
@@ -284,7 +287,7 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
           u32x2_t hh, mm, ll;
-          split3(__builtin_bit_cast(u32x4_t, s[qt][2 * c + x]), 1.0f, hh, mm, ll);
+          split3(__builtin_bit_cast(u32x4_t, s[qt][2 * c + x]), kSplitUp, hh, mm, ll);
           pf[0][qt][2 * x] = hh[0], pf[0][qt][2 * x + 1] = hh[1];
           pf[1][qt][2 * x] = mm[0], pf[1][qt][2 * x + 1] = mm[1];
           pf[2][qt][2 * x] = ll[0], pf[2][qt][2 * x + 1] = ll[1];
@@ -331,11 +334,7 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
 #pragma unroll
       for (int r = 0; r < 4; ++r) chk = __builtin_fmaf(o_acc[qt][dt][r], 0.f, chk);
   }
-  bool odd = chk != chk;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    odd = odd || ((seen[e] & 0x7fffffffu) != 0 && (seen[e] & 0x70000000u) == 0);
-  const bool redo = __syncthreads_or(odd) != 0;
+  const bool redo = __syncthreads_or(odd || chk != chk) != 0;
   if (!wave_live) return;
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -351,7 +350,7 @@ __global__ __launch_bounds__(kAsThreads, QT == 1 ? 3 : 2) void attn_fwd_split_ke
     }
     const float l = column_sum(l_run[qt]);
     if (qi >= Tq) continue;
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const float inv = (l > 0.f ? 1.0f / l : 0.f) * (redo ? 1.0f : kSplitDown * kSplitDown);
     float* orow = O + b * o_sb + h * o_sh + qi * o_st;
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt) {

@@ -76,3 +76,47 @@ def test_split_attention_tiny_values(gpu, scale):
     out, ref = cutile_causal_attention(q, k, v, H).double(), exact(q, k, v)
     col = (out - ref).norm(dim=2) / ref.norm(dim=2)
     assert col.max() <= TOL, col.max()
+
+
+def row_err(out, ref):
+    """Largest error of a row over the row's norm."""
+    return ((out.double() - ref).norm(dim=-1) / ref.norm(dim=-1)).max()
+
+
+# Elements of Q and K of inverse scales: in every column, or in every second one
+# (an ordinary value beside each small one).  Ordinary scores, so TOL holds.
+@pytest.mark.parametrize("step", [1, 2])
+@pytest.mark.parametrize("e", [-125, -123, -100, -90, -70, 70, 90, 100, 115, 123, 125])
+def test_split_attention_inverse_scales(gpu, e, step):
+    q, k, v = (randn(gpu, 1, 2, 150, 64, seed=i) for i in range(3))
+    q[..., ::step] *= 2.0 ** e
+    k[..., ::step] *= 2.0 ** -e
+    out = cutile_causal_attention(q, k, v, 2)
+    assert (out.double() - exact(q, k, v)).abs().max() <= TOL
+
+
+# Early rows see small values of V alone; the same columns are ordinary for
+# later keys.  Relative to each row: the bound for |v| <= 5 over a row's norm of
+# about 8 / sqrt(150).
+@pytest.mark.parametrize("e", [100, 115, 120, 125])
+def test_split_attention_tiny_values_before_others(gpu, e):
+    q, k, v = (randn(gpu, 1, 2, 150, 64, seed=i) for i in range(3))
+    v[:, :, :70] *= 2.0 ** -e
+    out, ref = cutile_causal_attention(q, k, v, 2), exact(q, k, v)
+    assert row_err(out[:, :, :70], ref[:, :, :70]) <= TOL
+    assert row_err(out[:, :, 70:], ref[:, :, 70:]) <= TOL
+
+
+# Small probabilities beside large ones whose values are zero: the result is the
+# small ones' alone.  fp32 rounds the exponent of 2^-g to 2^-17 absolute (2^-18
+# in the score, 2^-18 in its scaling), 8 such errors of 0.7 * 2^-17 each.
+@pytest.mark.parametrize("g", [60, 100, 115, 120, 124])
+def test_split_attention_tiny_probabilities(gpu, g):
+    q, k, v = (randn(gpu, 1, 1, 100, 64, seed=i) for i in range(3))
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    q[..., 1:] *= 1e-3
+    k[..., ::2, 0] = -g * math.log(2.0) * 8   # every second key: 2^-g of the others
+    v[..., ::2, :] *= 2.0 ** 100
+    v[..., 1::2, :] = 0.0
+    out, ref = cutile_causal_attention(q, k, v, 1), exact(q, k, v)
+    assert row_err(out[:, :, 1:], ref[:, :, 1:]) <= 8 * 2.0 ** -17
