@@ -27,7 +27,9 @@ extern "C" int cgpt_forward(const int64_t* a, const int64_t* layers, float scale
   const int64_t c_layer = a[29], csb = a[30], csh = a[31], cst = a[32], t_max = a[33];
   const int t_qkv = static_cast<int>(a[34]), t_proj = static_cast<int>(a[35]);
   const int t_fc = static_cast<int>(a[36]), t_mlp = static_cast<int>(a[37]);
-  if (B <= 0 || T <= 0 || D <= 0 || H <= 0 || n_layer <= 0 || D % H != 0) return CGPT_EINVAL;
+  // No sequences or no positions: nothing to do, as for every launch below; but
+  // no position is no last position.
+  if (B < 0 || T < 0 || (last && T == 0) || D <= 0 || H <= 0 || n_layer <= 0 || D % H != 0) return CGPT_EINVAL;
   if (act != CGPT_F32 && act != CGPT_BF16) return CGPT_EDTYPE;
   const int64_t M = B * T, hd = D / H, es = act == CGPT_F32 ? 4 : 2;
   const uint8_t* q = static_cast<const uint8_t*>(qkv);
