@@ -262,14 +262,25 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        // Lane l supplies row l % 32 and k + l / 32 of both operands.
+        // Lane l supplies row l % 32 of both operands, and of every 2 KV k the KV
+        // from KV (l / 32) on (any one order of k serves).  Four k a load, one
+        // where the accumulators leave no registers for it (one -> four, a NaN in
+        // every tile: 4096 x 3072 x 768 1088 -> 400 us, 87 rows of it 177 -> 57).
+        constexpr int KV = TM * TN > 4 ? 1 : 4;
         const float* pa = A + static_cast<int64_t>(min(m0 + wm0 + i * 32 + r32, M - 1)) * lda;
         const float* pw = W + static_cast<int64_t>(min(n0 + wn0 + j * 32 + r32, N - 1)) * ldw;
         f32x16_t t;
 #pragma unroll
         for (int r = 0; r < 16; ++r) t[r] = 0.f;
-        for (int k = 0; k < K; k += 2)
-          t = __builtin_amdgcn_mfma_f32_32x32x2f32(pw[k + g], pa[k + g], t, 0, 0, 0);
+        for (int k0 = 0; k0 < K; k0 += 2 * KV) {
+          const int k = k0 + KV * g, at = min(k, K - KV);
+          float va[KV], vw[KV];
+#pragma unroll
+          for (int e = 0; e < KV; ++e) va[e] = pa[at + e], vw[e] = pw[at + e];
+#pragma unroll
+          for (int e = 0; e < KV; ++e)
+            t = __builtin_amdgcn_mfma_f32_32x32x2f32(k < K ? vw[e] : 0.f, k < K ? va[e] : 0.f, t, 0, 0, 0);
+        }
         acc[i][j] = t;
       }
   }
