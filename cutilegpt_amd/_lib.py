@@ -70,13 +70,18 @@ SIGNATURES = {
                                          _I64, _F, _I, _I, _I, _I, _P]),
     "cgpt_kv_store": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                            _I64, _I64, _I64, _I64, _I64, _I64, _I, _P]),
-    "cgpt_forward": (_I, [_P, _P, _F, _F, _P]),
+    "cgpt_forward": (_I, [_P, _I64, _P, _F, _F, _P, _P, _P]),
     "cgpt_argmax": (_I, [_P, _I64, _I64, _I64, _I, _P, _P, _I64, _P, _P]),
     "cgpt_partials_bias_act": (_I, [_P, _I64, _I64, _I64, _P, _I, _P, _I64, _I64, _I64, _I, _I,
                                     _P]),
 }
 
 ABI_VERSION = 1
+
+# cgpt_forward's launches, by tag, and its probe (tag, start) -> 0 to go on.
+FORWARD_TAGS = ("embedding", "gemm_qkv", "kv_store", "attention", "gemm_proj", "ln", "gemm_fc_gelu",
+                "gemm_mlp_proj", "lm_head")
+FORWARD_PROBE = ctypes.CFUNCTYPE(_I, _I, _I)
 
 
 class KernelLibraryError(RuntimeError):

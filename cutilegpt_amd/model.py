@@ -189,16 +189,10 @@ class CutileGPT:
         cfg = self.config
         assert T <= cfg.block_size, f"Sequence length {T} > block_size {cfg.block_size}"
         idx = self._prepare_idx(idx)
-        lib = _lib.load()
-        chk = _lib.check
-        W = self.weights
-        D, H, V = cfg.n_embd, cfg.n_head, cfg.vocab_size
-        hd = D // H
+        D, V = cfg.n_embd, cfg.vocab_size
         M = B * T
         dev = self.device
         act = self.dtype
-        ac = _DT[act]
-        f32 = _lib.CGPT_F32
         s = torch.cuda.current_stream(dev).cuda_stream
         if self._err is None:
             self._err = torch.zeros(1, dtype=torch.int32, device=dev)
@@ -211,88 +205,15 @@ class CutileGPT:
         Vp = self._head_pad.shape[0]
         logits = (torch.empty((M, Vp), dtype=self.logits_dtype, device=dev)
                   if logits_out is None else None)
-        px, ph, pq, pa, pf = (t.data_ptr() for t in (x, h, qkv, att, f))
-
-        scale = 1.0 / math.sqrt(hd)
-        if probe is None:
-            # The whole launch sequence in one native call.
-            self._launch_forward(lib, idx, (px, ph, pq, pa, pf), cache, logits, logits_out, s)
-            return logits_out if logits_out is not None else logits[:, :V].view(B, T, V)
-
-        mark = probe
-
-        def gemm(tag, a_ptr, w, b, c_ptr, n, k, epi, out_code):
-            t = gemm_tile(ac, M, n, k)
-            mark(tag, True)
-            chk(lib.cgpt_gemm(a_ptr, w.data_ptr(), None if b is None else b.data_ptr(), c_ptr,
-                              M, n, k, k, w.stride(0), n, ac, ac, out_code, epi, t, s), tag)
-            mark(tag, False)
-
-        def ln(wk):
-            # h = LayerNorm(x); x itself is left as it is.
-            mark("ln", True)
-            chk(lib.cgpt_add_layernorm(px, None, None, W[wk + ".weight"].data_ptr(),
-                                       W[wk + ".bias"].data_ptr(), ph, M, D, 1e-5, f32, f32, ac,
-                                       ac, s), "layernorm")
-            mark("ln", False)
-
-        # x = wte[idx] + wpe[pos] and h = ln_1(x) of layer 0 in one pass.
-        mark("embedding", True)
-        chk(lib.cgpt_embedding_layernorm(idx.data_ptr(), W["wte"].data_ptr(), W["wpe"].data_ptr(),
-                                         None, px, W["h.0.ln_1.weight"].data_ptr(),
-                                         W["h.0.ln_1.bias"].data_ptr(), ph, M, T, D, V, 0,
-                                         cfg.block_size, 1e-5, ac, ac, self._err.data_ptr(), s),
-            "embedding_layernorm")
-        mark("embedding", False)
-        st_qkv = (T * 3 * D, hd, 3 * D)
-        st_o = (T * D, hd, D)
-        for i in range(cfg.n_layer):
-            p = f"h.{i}."
-            gemm("gemm_qkv", ph, W[p + "attn.c_attn.weight"], W[p + "attn.c_attn.bias"], pq,
-                 3 * D, D, _lib.EPI_BIAS, ac)
-            esz = qkv.element_size()
-            if cache is not None:
-                csb, csh, cst = cache.strides()
-                chk(lib.cgpt_kv_store(pq + D * esz, pq + 2 * D * esz, cache.k[i].data_ptr(),
-                                      cache.v[i].data_ptr(), B, H, T, hd, 0, cache.t_max,
-                                      *st_qkv, *st_qkv, csb, csh, cst, ac, s), "kv_store")
-            mark("attention", True)
-            chk(lib.cgpt_attention_fwd(pq, pq + D * esz, pq + 2 * D * esz, pa, B, H, T, T, hd,
-                                       *st_qkv, *st_qkv, *st_qkv, *st_o, scale, 1, ac, s),
-                "attention")
-            mark("attention", False)
-            # x += att Wo^T + b (residual add in the GEMM epilogue, in place)
-            gemm("gemm_proj", pa, W[p + "attn.c_proj.weight"], W[p + "attn.c_proj.bias"], px,
-                 D, D, _lib.EPI_BIAS_RESID, f32)
-            ln(p + "ln_2")
-            gemm("gemm_fc_gelu", ph, W[p + "mlp.c_fc.weight"], W[p + "mlp.c_fc.bias"], pf,
-                 4 * D, D, _lib.EPI_BIAS_GELU, ac)
-            gemm("gemm_mlp_proj", pf, W[p + "mlp.c_proj.weight"], W[p + "mlp.c_proj.bias"], px,
-                 D, 4 * D, _lib.EPI_BIAS_RESID, f32)
-            ln("ln_f" if i + 1 == cfg.n_layer else f"h.{i + 1}.ln_1")
-        if logits_out is not None:
-            # Last position of each sequence: rows b*T + T-1 of h, stride T*D.
-            mark("lm_head", True)
-            chk(lib.cgpt_gemm(ph + (T - 1) * D * h.element_size(), W["lm_head.weight"].data_ptr(),
-                              None, logits_out.data_ptr(), B, V, D, T * D,
-                              W["lm_head.weight"].stride(0), V, ac, ac, _DT[logits_out.dtype],
-                              _lib.EPI_NONE, _lib.TILE_AUTO, s), "lm_head")
-            mark("lm_head", False)
-            return logits_out
+        self._launch_forward(idx, (x, h, qkv, att, f), cache, logits, logits_out, probe, s)
         # Padded head: logits rows have stride Vp; the returned (B, T, V) tensor
         # is a view of the first V columns.
-        mark("lm_head", True)
-        head = self._head_pad
-        chk(lib.cgpt_gemm(ph, head.data_ptr(), None, logits.data_ptr(), M, Vp, D, D, head.stride(0),
-                          Vp, ac, ac, _DT[self.logits_dtype], _lib.EPI_NONE,
-                          gemm_tile(ac, M, Vp, D), s), "lm_head")
-        mark("lm_head", False)
-        return logits[:, :V].view(B, T, V)
+        return logits_out if logits_out is not None else logits[:, :V].view(B, T, V)
 
-    def _launch_forward(self, lib, idx: torch.Tensor, bufs, cache, logits: Optional[torch.Tensor],
-                        logits_out: Optional[torch.Tensor], stream: int) -> None:
-        """``_forward``'s launches through ``cgpt_forward``, from the weights as
-        the model holds them at this call."""
+    def _launch_forward(self, idx: torch.Tensor, bufs, cache, logits: Optional[torch.Tensor],
+                        logits_out: Optional[torch.Tensor], probe, stream: int) -> None:
+        """``_forward``'s launches, one native call (``cgpt_forward``), from the
+        weights as the model holds them at this call."""
         cfg, W = self.config, self.weights
         B, T = idx.shape
         D, V, M = cfg.n_embd, cfg.vocab_size, B * T
@@ -309,7 +230,7 @@ class CutileGPT:
                   *cache.strides(), cache.t_max)
         vals = [B, T, D, cfg.n_head, V, cfg.n_layer, cfg.block_size, ac, idx.data_ptr(),
                 W["wte"].data_ptr(), W["wpe"].data_ptr(), W["ln_f.weight"].data_ptr(),
-                W["ln_f.bias"].data_ptr(), *bufs, self._err.data_ptr(), head.data_ptr(), head.stride(0),
+                W["ln_f.bias"].data_ptr(), *(t.data_ptr() for t in bufs), self._err.data_ptr(), head.data_ptr(), head.stride(0),
                 n_head, out.data_ptr(), out.stride(0), _DT[out.dtype], head_tile,
                 int(logits_out is not None), *kv, gemm_tile(ac, M, 3 * D, D), gemm_tile(ac, M, D, D),
                 gemm_tile(ac, M, 4 * D, D), gemm_tile(ac, M, D, 4 * D)]
@@ -319,9 +240,24 @@ class CutileGPT:
             layers += [w.data_ptr() for w in ws]
             layers += [ws[2].stride(0), ws[4].stride(0), ws[8].stride(0), ws[10].stride(0)]
         layers += [0, 0]  # the entry past the last layer is never dereferenced
-        _lib.check(lib.cgpt_forward((ctypes.c_int64 * len(vals))(*vals),
-                                    (ctypes.c_int64 * len(layers))(*layers),
-                                    1.0 / math.sqrt(D // cfg.n_head), 1e-5, stream), "forward")
+        failed, raised = ctypes.c_int(-1), []
+
+        def call_probe(tag: int, start: int) -> int:
+            try:
+                probe(_lib.FORWARD_TAGS[tag], bool(start))
+            except BaseException as e:  # raised again below: it cannot pass the native frames
+                raised.append(e)
+            return len(raised)
+
+        hook = None if probe is None else _lib.FORWARD_PROBE(call_probe)
+        rc = _lib.load().cgpt_forward((ctypes.c_int64 * len(vals))(*vals), len(vals),
+                              (ctypes.c_int64 * len(layers))(*layers), 1.0 / math.sqrt(D // cfg.n_head), 1e-5,
+                              None if hook is None else ctypes.cast(hook, ctypes.c_void_p),
+                              ctypes.byref(failed), stream)
+        if raised:
+            raise raised[0]
+        if rc != 0:
+            _lib.check(rc, "forward" if failed.value < 0 else f"forward: {_lib.FORWARD_TAGS[failed.value]}")
 
     def input_errors(self) -> bool:
         """True if any forward so far saw a token id outside the vocabulary

@@ -375,15 +375,33 @@ int cgpt_attention_decode_partials(const float* qkv_partials, int64_t n_parts,
  * projection with the residual and the next LayerNorm, then the LM head: the
  * launches of the entry points above, in order, on `stream`.
  *
- * a: [0] B, T, D, H, V, n_layer, block_size, act dtype; [8] idx (int64, B x T),
+ * a, CGPT_FORWARD_ARGS values (n_a, refused otherwise): [0] B, T, D, H, V, n_layer, block_size, act dtype; [8] idx (int64, B x T),
  * wte, wpe, ln_f weight, ln_f bias; [13] x (fp32, B T x D), h, qkv, att, f (act
  * dtype), err flag; [19] head weight, its row stride, its rows; [22] logits,
  * row stride, dtype, tile, last (1: only each sequence's last position);
  * [27] k cache, v cache (0: none), bytes a layer, element strides (batch, head,
  * time), t_max; [34] tiles of the QKV, projection, c_fc and MLP projection GEMMs.
  * layers: 16 values each: ln_1 weight and bias, then weight and bias of c_attn and
- * attn c_proj, of ln_2, of c_fc and mlp c_proj, and the four weights' row strides. */
-int cgpt_forward(const int64_t* a, const int64_t* layers, float scale, float eps, void* stream);
+ * attn c_proj, of ln_2, of c_fc and mlp c_proj, and the four weights' row strides;
+ * after the last layer two values more, which are not read through.
+ * probe (may be NULL): called with the launch's tag and 1 right before, 0 right
+ * after each launch; a nonzero result ends the call (CGPT_EINVAL).
+ * failed (may be NULL): on an error, the tag of the launch it came from
+ * (CGPT_FWD_ARGS: the arguments here). */
+#define CGPT_FORWARD_ARGS 38
+#define CGPT_FWD_ARGS (-1)
+#define CGPT_FWD_EMBEDDING 0
+#define CGPT_FWD_QKV 1
+#define CGPT_FWD_KV_STORE 2
+#define CGPT_FWD_ATTENTION 3
+#define CGPT_FWD_PROJ 4
+#define CGPT_FWD_LN 5
+#define CGPT_FWD_FC 6
+#define CGPT_FWD_MLP_PROJ 7
+#define CGPT_FWD_HEAD 8
+typedef int (*cgpt_probe_fn)(int tag, int start);
+int cgpt_forward(const int64_t* a, int64_t n_a, const int64_t* layers, float scale, float eps,
+                 cgpt_probe_fn probe, int* failed, void* stream);
 
 /*
  * Copy T positions of keys and values ((b, h, t, d) at base + b*sb + h*sh + t*st
