@@ -57,6 +57,30 @@ def test_layernorm_gemm(gpu, M, N, K, n_in):
     assert ((out.sum(0).double() - ref).norm() / ref.norm()) <= 1e-3
 
 
+# Up to 1024 columns a wave of either kernel sums the same 256 of a row, in the
+# same order, so the operand is the same bit for bit.
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("N,K,n_in", [(4, 64, 1), (132, 128, 3), (768, 768, 12), (3072, 1024, 16)])
+def test_layernorm_gemm_equals_two_launches(gpu, M, N, K, n_in):
+    lib = _lib.load()
+    assert lib.cgpt_decode_fused_ok(M, N, K, K, n_in, 1)
+    t = make(gpu, N + K + n_in, M, N, K, n_in)
+    ns = plan(M, N, K)
+    out, two = torch.empty(ns, M, N, device=gpu), torch.empty(ns, M, N, device=gpu)
+    x2, x3, h = torch.empty(M, K, device=gpu), torch.empty(M, K, device=gpu), torch.empty(M, K, dtype=BF16, device=gpu)
+    _lib.check(lib.cgpt_gemm_partials_ln(
+        t["x"].data_ptr(), t["parts"].data_ptr(), n_in, M * K, K, t["bias"].data_ptr(), x2.data_ptr(),
+        t["gamma"].data_ptr(), t["beta"].data_ptr(), 1e-5, t["w"].data_ptr(), out.data_ptr(), M, N, K,
+        K, N, ns, stream(gpu)), "ln")
+    _lib.check(lib.cgpt_add_layernorm_partials(
+        t["x"].data_ptr(), t["parts"].data_ptr(), n_in, M * K, K, t["bias"].data_ptr(), x3.data_ptr(),
+        t["gamma"].data_ptr(), t["beta"].data_ptr(), h.data_ptr(), M, K, 1e-5, _lib.CGPT_F32, _lib.CGPT_F32,
+        _lib.CGPT_BF16, _lib.CGPT_BF16, stream(gpu)), "add_ln")
+    _lib.check(lib.cgpt_gemm_partials(h.data_ptr(), t["w"].data_ptr(), two.data_ptr(), M, N, K, K, K, N,
+                                      ns, _lib.CGPT_BF16, stream(gpu)), "partials")
+    assert torch.equal(x2, x3) and torch.equal(out, two)
+
+
 @pytest.mark.parametrize("M", [1, 2])
 @pytest.mark.parametrize("N,K,n_in", [(4, 64, 1), (132, 192, 3), (768, 3072, 5), (1600, 2560, 16),
                                       (512, 2048, 9)])
