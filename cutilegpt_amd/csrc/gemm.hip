@@ -1620,7 +1620,9 @@ static int launch_tile(int tile, const void* a, const void* w, const void* bias,
 // most); the choice it replaces (tiles counted per CU) took 1.22 (2.44), mostly
 // where few tiles leave the CUs waiting: 70 x 1600 x 6400 36.4 -> 14.9 us,
 // 591 x 2304 x 768 8.9 -> 8.4, 2700 x 768 x 3072 39 -> 26, 4096 x 2304 x 768
-// 26 -> 19.3, 4096 x 768 x 3072 with the residual 43 -> 33.
+// 26 -> 19.3, 4096 x 768 x 3072 with the residual 43 -> 33.  The timings behind
+// the fit were not kept; `python -m cutilegpt_amd.tune --check` times TILE_AUTO
+// against every tile with a public id over such a set.
 struct TileCost {
   int id, bm, bn, blocks;
   float start, step[3], end[3], fill, out, gelu, ops;
@@ -1688,7 +1690,9 @@ static int cheapest_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi,
 // for as long as a full one: 1000 x 50257 x 768 (bf16 out) is 788 tiles, three
 // rounds and 20 tiles, 116.4 -> 102.9 us in two launches; 1000 x 50304 x 1600
 // (fp32 out) 186.4 -> 164.0, 300 x 50257 x 1600 101.1 -> 88.0, 3000 x 50304 x
-// 1600 499 -> 479.  The CUs drift apart over many rounds and share the last one
+// 1600 499 -> 479.  An explicit tile id is always one launch: the heads that the
+// caller's table (tiles.py) gives tile 16 do not come here, the last of these
+// among them.  The CUs drift apart over many rounds and share the last one
 // better than predicted: heads with less than 2.5% to gain ran 0.97 to 1.03
 // times as fast (4096 x 50304 x 768, 0.8% predicted, 342 -> 352), those above
 // it 1.01 to 1.18.  Narrower products gained and lost (0.94 to 1.07).
@@ -1891,7 +1895,7 @@ static int launch_epi(int epi, int tile, const void* a, const void* w, const voi
       default:
         return CGPT_EINVAL;
     }
-    }
+  }
 }
 
 }  // namespace cgpt

@@ -43,7 +43,10 @@ Anything else takes the library's own choice (``TILE_AUTO``): for 16-bit inputs
 the tile whose predicted launch time is lowest (``tile_cost`` in
 ``csrc/gemm.hip``; the tiles of ``csrc/gemm_kgroup.hip``, which have no id here,
 among them), for the exact M rather than its bucket, which is why the table
-holds only the LM heads and products whose best tile is the same over a bucket.
+holds only the LM heads and products whose best tile was the same over a bucket.
+A table entry is one launch of its tile; only ``TILE_AUTO`` splits off the last
+columns of a wide product whose last round is nearly empty, so the heads listed
+here are not split.
 For the residual epilogue (attn / MLP c_proj into the fp32 residual stream) a
 tile id picks between the slab kernel (14), the small pipeline tiles (17-19)
 and the register-staged tiles.
@@ -61,8 +64,8 @@ def m_bucket(m: int) -> int:
     return 1 << max(0, (int(m) - 1).bit_length())
 
 
-# (dtype code, M bucket, N, K) -> tile id, from the sweep (TFLOP/s by kernel time of the
-# winner, inputs hot; attn/MLP c_proj with the residual epilogue, fp32 out).
+# (dtype code, M bucket, N, K) -> tile id, from the sweep of the tiles with ids (TFLOP/s by
+# kernel time of the winner, inputs hot; attn c_proj with the residual epilogue, fp32 out).
 _B = _lib.CGPT_BF16
 TABLE: Dict[Tuple[int, int, int, int], int] = {
     # GPT-2 124M prefill, M = 16 x 1024

@@ -16,6 +16,11 @@ launch overhead out of short kernels' times).  The residual-epilogue shapes (att
 c_proj: C += A W^T + bias into the fp32 residual stream) sweep the tiles that
 epilogue runs on: the register-staged tiles 0-4, the slab kernel (14) and the
 small pipeline tiles (17-19).
+
+``--check`` times ``TILE_AUTO`` instead, against every tile above, over the four
+layer products of several widths and row counts, and prints each one's ratio to
+the best of them and the geometric mean (``TILE_AUTO`` also has tiles without an
+id, those of ``csrc/gemm_kgroup.hip``: ratios below one are theirs).
 Needs a GPU.
 """
 
@@ -23,6 +28,7 @@ from __future__ import annotations
 
 import argparse
 import json
+import math
 import sys
 from typing import Dict, List, Tuple
 
@@ -36,22 +42,28 @@ CONFIGS: Dict[str, Tuple[int, int]] = {
 }
 VOCAB_PAD = 50304
 RESID_TILES = [0, 1, 2, 3, 4, 14, 17, 18, 19]
+# --check: widths and rows (a short prompt to a full batch).
+CHECK_D = (256, 512, 768, 1024, 1600)
+CHECK_M = (70, 200, 591, 1500, 2700, 4096, 16384)
+
+
+def layer_shapes(d: int, m: int) -> List[Tuple[str, int, int, int, int, int]]:
+    """The four layer products of ``shapes`` for a width and a row count."""
+    bf, f32 = _lib.CGPT_BF16, _lib.CGPT_F32
+    return [("c_attn", m, 3 * d, d, _lib.EPI_BIAS, bf),
+            ("attn_c_proj", m, d, d, _lib.EPI_BIAS_RESID, f32),
+            ("c_fc_gelu", m, 4 * d, d, _lib.EPI_BIAS_GELU, bf),
+            ("mlp_c_proj", m, d, 4 * d, _lib.EPI_BIAS_RESID, f32)]
 
 
 def shapes(name: str) -> List[Tuple[str, int, int, int, int, int]]:
     """(tag, M, N, K, epilogue, out dtype) of every GEMM in the forward."""
     d, m = CONFIGS[name]
-    bf, f32 = _lib.CGPT_BF16, _lib.CGPT_F32
-    return [
-        ("c_attn", m, 3 * d, d, _lib.EPI_BIAS, bf),
-        ("attn_c_proj", m, d, d, _lib.EPI_BIAS_RESID, f32),
-        ("c_fc_gelu", m, 4 * d, d, _lib.EPI_BIAS_GELU, bf),
-        ("mlp_c_proj", m, d, 4 * d, _lib.EPI_BIAS_RESID, f32),
-        ("lm_head", m, VOCAB_PAD, d, _lib.EPI_NONE, f32),
-    ]
+    return layer_shapes(d, m) + [("lm_head", m, VOCAB_PAD, d, _lib.EPI_NONE, _lib.CGPT_F32)]
 
 
-def sweep(name: str, iters: int, warmup: int, out=sys.stdout):
+def sweep(name: str, problems, iters: int, warmup: int, auto: bool = False, out=sys.stdout):
+    """Winner of each of ``problems`` and every timing; ``auto``: ``TILE_AUTO``'s too."""
     import torch
 
     lib = _lib.load()
@@ -61,13 +73,15 @@ def sweep(name: str, iters: int, warmup: int, out=sys.stdout):
     g = torch.Generator(device=dev).manual_seed(0)
     winners = {}
     rows = []
-    for tag, m, n, k, epi, oc in shapes(name):
+    for tag, m, n, k, epi, oc in problems:
         a = (torch.randn(m, k, device=dev, generator=g) * 0.5).to(torch.bfloat16)
         w = (torch.randn(n, k, device=dev, generator=g) * 0.02).to(torch.bfloat16)
         b = (torch.randn(n, device=dev, generator=g) * 0.02).to(torch.bfloat16)
         c = torch.zeros(m, n, device=dev,
                         dtype=torch.float32 if oc == _lib.CGPT_F32 else torch.bfloat16)
         tiles = RESID_TILES if epi == _lib.EPI_BIAS_RESID else list(range(ntiles))
+        if auto:
+            tiles = [_lib.TILE_AUTO] + tiles
         fl = 2.0 * m * n * k
         best = None
         for t in tiles:
@@ -96,9 +110,10 @@ def sweep(name: str, iters: int, warmup: int, out=sys.stdout):
             del graph
             ms = e0.elapsed_time(e1) / iters
             rows.append((name, tag, m, n, k, t, ms, fl / ms / 1e9))
-            print(f"{name:7s} {tag:12s} M={m:6d} N={n:6d} K={k:5d} tile {t:2d}: "
-                  f"{ms * 1e3:9.1f} us {fl / ms / 1e9:7.1f} TFLOP/s", file=out, flush=True)
-            if best is None or ms < best[1]:
+            if out is not None:
+                print(f"{name:7s} {tag:12s} M={m:6d} N={n:6d} K={k:5d} tile {t:2d}: "
+                      f"{ms * 1e3:9.1f} us {fl / ms / 1e9:7.1f} TFLOP/s", file=out, flush=True)
+            if t != _lib.TILE_AUTO and (best is None or ms < best[1]):
                 best = (t, ms)
         if epi == _lib.EPI_BIAS_RESID and c.dtype == torch.float32:
             c.zero_()  # keep the residual buffer finite after many in-place adds
@@ -114,10 +129,27 @@ def main(argv=None) -> int:
     ap.add_argument("--configs", nargs="+", default=sorted(CONFIGS), choices=sorted(CONFIGS))
     ap.add_argument("--iters", type=int, default=10)
     ap.add_argument("--warmup", type=int, default=3)
+    ap.add_argument("--check", action="store_true", help="TILE_AUTO against every tile")
     args = ap.parse_args(argv)
+    if args.check:
+        logs = []
+        for d in CHECK_D:
+            for m in CHECK_M:
+                _, rows = sweep(f"d{d}", layer_shapes(d, m), args.iters, args.warmup, auto=True, out=None)
+                for tag in dict.fromkeys(r[1] for r in rows):
+                    us = {r[5]: r[6] * 1e3 for r in rows if r[1] == tag}
+                    mine = us.pop(_lib.TILE_AUTO)
+                    best = min(us, key=us.get)
+                    logs.append(math.log(mine / us[best]))
+                    _, _, M, N, K = next(r for r in rows if r[1] == tag)[:5]
+                    print(f"{tag:12s} M={M:6d} N={N:5d} K={K:5d}: auto {mine:7.1f} us, best tile {best:2d} "
+                          f"{us[best]:7.1f} us, ratio {mine / us[best]:.3f}", flush=True)
+        print(f"geometric mean over {len(logs)} problems {math.exp(sum(logs) / len(logs)):.3f}, "
+              f"largest {math.exp(max(logs)):.3f}", flush=True)
+        return 0
     table = {}
     for name in args.configs:
-        winners, _ = sweep(name, args.iters, args.warmup)
+        winners, _ = sweep(name, shapes(name), args.iters, args.warmup)
         for (m, n, k), (tag, t, ms, tf) in winners.items():
             print(f"winner {name:7s} {tag:12s} ({m}, {n}, {k}): tile {t} "
                   f"{ms * 1e3:.1f} us {tf:.1f} TFLOP/s", flush=True)
