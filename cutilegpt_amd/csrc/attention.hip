@@ -724,7 +724,7 @@ static int launch_attn(const void* q, const void* k, const void* v, void* o, int
   const bool small = blocks128 < 4 * static_cast<int64_t>(attn_num_cus());
   const int bq = small ? 64 : 128;
   // fp32 at head_dim 64: split operands on the bf16 matrix cores, 8x12x512
-  // 50 -> 33 us, 16x12x1024 270 -> 165 (64 queries a block: 195), 1x12x87
+  // 45 -> 30 us, 16x12x1024 255 -> 160 (64 queries a block: 195), 1x12x87
   // 8.9 -> 7.7, against the fp32 MFMA; the error against float64 is below half
   // of it (8x12x512: 2.8e-7 -> 1.1e-7).  The other head_dims' models are small.
   if constexpr (sizeof(T) == 4 && HD == 64) {

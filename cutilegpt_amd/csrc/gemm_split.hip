@@ -85,8 +85,8 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, BM * BN == 128 * 128 && KG == 
   const uint8_t* ab = reinterpret_cast<const uint8_t*>(A + static_cast<int64_t>(m0) * lda);
   const uint8_t* wb = reinterpret_cast<const uint8_t*>(W + static_cast<int64_t>(n0) * ldw);
 
-  // Byte offsets of this thread's rows in the tile (the host keeps a tile's
-  // rows below 2 GiB); rows past the matrix are clamped to the last one
+  // Byte offsets of this thread's rows in the tile, unsigned: the host keeps a
+  // tile's rows within 4 GiB (256 rows less than 2^22 floats apart); rows past the matrix are clamped to the last one
   // (loaded, never stored).
   uint32_t ao[A_LD], wo[W_LD];
 #pragma unroll

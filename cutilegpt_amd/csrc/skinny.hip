@@ -629,7 +629,7 @@ struct DecProIn {
   const bf16_t* beta;
   float eps;
 };
-constexpr int kProMaxRows = 2;
+constexpr int kProMaxRows = 2;  // as many as were built and timed, not a measured limit
 
 #if defined(__HIP_DEVICE_COMPILE__)
 __device__ __forceinline__ void bf16x4_to_f32(const u32x2_t& w, float* v) {
@@ -1187,7 +1187,7 @@ int launch_gemm_partials(bool bf16_in, const void* a, const void* w, float* part
 // Whether gemm_decode_pro_kernel takes a product: N a multiple of 4, K whole
 // double slabs (a LayerNorm row at most 2048), the decode form's own plan for
 // the split with at most five double slabs a chunk (the pass's registers), and
-// at most eight partials a row for two rows, sixteen for one.
+// at most kSkMaxSplit (16) partials a row, for one row as for two.
 bool decode_pro_ok(bool ln, int M, int N, int K, int64_t ldw, int n_parts) {
   DecodePlan dp;
   return M >= 1 && M <= kProMaxRows && N % 4 == 0 && K % 64 == 0 && (!ln || K <= 2048) && n_parts >= 1 &&

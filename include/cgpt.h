@@ -130,8 +130,10 @@ int cgpt_partials_bias_act(const float* partials, int64_t n_parts, int64_t part_
  * with leading dimension ldw — the nn.Linear / cutileGPT `weight` layout, so no
  * transposed copy is needed — C row-major with leading dimension ldc.
  * in_dtype is the type of A and W (CGPT_BF16 -> bf16 MFMA, CGPT_F16 -> fp16
- * MFMA, CGPT_F32 -> fp32 MFMA); accumulation is fp32; bias (bias_dtype) is
- * added in fp32; C is written as out_dtype.  bias_dtype and out_dtype are
+ * MFMA, CGPT_F32 -> three bf16 parts of every value, six bf16 MFMAs a product,
+ * with fp32's precision for every fp32 value; the fp32 MFMA for the skinny and
+ * the element-load kernel); accumulation is fp32; bias (bias_dtype) is added in
+ * fp32; C is written as out_dtype.  bias_dtype and out_dtype are
  * CGPT_F32 or the 16-bit type of the inputs' family (CGPT_F16 with fp16 inputs,
  * CGPT_BF16 otherwise).  Any K >= 1, lda >= K, ldw >= K and element-aligned
  * pointers: problems with K, lda and ldw multiples of 8 (16-bit) or 4 (fp32)
@@ -147,10 +149,12 @@ int cgpt_partials_bias_act(const float* partials, int64_t n_parts, int64_t part_
  * With CGPT_EPI_BIAS_RESID (C += A W^T + bias in place, C usually the fp32
  * residual stream), tile 14 asks for the slab kernel's residual ring, 17-19
  * for those 4-wave pipeline tiles, a register-staged id (bf16 / fp16 0-4,
- * fp32 0-1) for that tile, and any other id means CGPT_TILE_AUTO.  A persistent launch (bf16 tile >= 5) over a
- * weight matrix of at least 32 MiB with M >= 1024 first reads W once on the
- * same stream (one extra kernel) so that the launch's repeated W band fetches
- * are served from the memory-side cache.
+ * fp32 0-1) for that tile, and any other id means CGPT_TILE_AUTO.  A persistent
+ * launch (bf16 tile >= 5) over a weight matrix of at least 32 MiB with M >= 1024
+ * first reads W once on the same stream (one extra kernel) so that the launch's
+ * repeated W band fetches are served from the memory-side cache.  With
+ * CGPT_TILE_AUTO a 16-bit product of 16384 columns and more may be two launches,
+ * the last columns in smaller tiles; an explicit id never is.
  * Replaces cutile_linear / cutile_linear_bias, cutile_gpt/kernels/linear.py:112-222
  * (kernels :37-109); CGPT_EPI_BIAS_GELU also absorbs cutile_gelu at
  * cutile_gpt/models/gpt.py:167.
