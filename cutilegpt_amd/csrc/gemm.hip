@@ -14,7 +14,7 @@
 //    which makes bias, GELU and the store 4-wide.
 //  * bf16 / fp16: v_mfma_f32_16x16x32_bf16 / _f16 (each lane supplies 8
 //    consecutive k); every 16-bit kernel is templated on the input type.
-//    fp32 (element loads only; aligned fp32 problems run gemm_split.hip): four
+//    fp32 (short K and element loads; other fp32 problems run gemm_split.hip): four
 //    v_mfma_f32_16x16x4_f32 per 16-byte fragment; lane group g supplies
 //    k = 4g + j to the j-th MFMA (any consistent permutation of the k axis
 //    leaves the dot product unchanged).
@@ -24,8 +24,8 @@
 //
 // Main loops:
 //  * gemm_kernel: global -> registers -> LDS double buffering (small 16-bit
-//    problems, any K multiple of 8; with element loads, any K, stride or
-//    alignment, fp32 included).
+//    problems, any K multiple of 8; fp32 of short K, mfma_f32 below; with
+//    element loads, any K, stride or alignment).
 //  * gemm_pipe_kernel / gemm_pipe_a3_kernel / gemm_slab_kernel: 16-bit
 //    direct-to-LDS multi-stage pipelines, persistent over tiles (see the
 //    comments above them).
@@ -106,8 +106,8 @@ __device__ __forceinline__ void store_block_remap(float* scr, TOut* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Register-staged double-buffered kernel (K % 8; with element loads any K and
-// fp32 too; the K tail of the last 128-byte row is zero-filled).
+// Register-staged double-buffered kernel (K % 8, fp32 K % 4; with element loads
+// any K; the K tail of the last 128-byte row is zero-filled).
 
 template <typename TIn, int BM, int BN, int WGM, int WGN, int EPI, typename TOut, bool EL = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(
@@ -1767,6 +1767,21 @@ static bool skinny_f32(int64_t M, int64_t N, int64_t K, bool far) {
   return M <= (N < kWideN && K >= 512 ? 16 : 32);
 }
 
+// Aligned fp32 problems that the fp32 MFMA's register-staged kernel takes instead
+// of the split one (us, fp32 MFMA against split, operands rotated past the caches):
+// with at most four 16-wide k stages the split kernel's pipelines never fill and
+// its blocks do not share a CU as well.  K = 32: 12000 x 96 7.2 / 12.6,
+// 4096 x 50257 472 / 583; K = 48: 7000 x 144 8.1 / 12.1, 1500 x 50257 212 / 232;
+// K = 64: 7000 x 192 8.6 / 12.9.  From K = 48 on the split kernel keeps few tiles
+// (1500 x 48 with the residual 7.3 / 6.3; not 16 rows and fewer, 4.8 / 5.4 in the
+// caches) and many whose rows take 16-byte stores (2700 x 50304 x 48 243 / 198).
+static bool mfma_f32(int M, int N, int K, bool vec_store) {
+  if (K > 64) return false;
+  auto tiles = [&](int t) { return static_cast<int64_t>((M + t - 1) / t) * ((N + t - 1) / t); };
+  if (K < 48 || M <= 16) return true;
+  return tiles(64) > 64 && !(vec_store && tiles(128) > 2 * num_cus());
+}
+
 // Residual epilogue (C += A W^T + bias).  `tile`: 14 = the slab kernel's
 // residual ring (16-bit inputs into fp32 C, at least 8 k64 steps, whole
 // 4-column groups, 32-bit offsets; otherwise as TILE_AUTO); 17-19 = that
@@ -1858,6 +1873,34 @@ static int launch_resid(int req_tile, const void* a, const void* w, const void* 
 #undef CGPT_RES_CFG
 }
 
+// fp32 without element loads: the fp32 MFMA (128x128 from two blocks a CU, else
+// 64x64) or the split kernel, whose tile ids 0 and 1 are.  far: rows too far
+// apart for the split kernel's 32-bit offsets.
+template <typename TOut>
+static int launch_f32(int epi, int tile, const void* a, const void* w, const void* bias, bool bias_bf16,
+                      void* c, int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, bool vec_store,
+                      bool far, hipStream_t s) {
+  const bool by_id = tile >= 0 && tile < kNumF32Tiles;
+  if (!far && (by_id || !mfma_f32(M, N, K, vec_store)))
+    return launch_gemm_split(epi, tile, a, w, bias, bias_bf16, c, sizeof(TOut) == 2, M, N, K, lda, ldw, ldc,
+                             vec_store, s);
+  const bool large = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128) >= 512;
+#define CGPT_F32_CASE(E)                                                                              \
+  case E:                                                                                             \
+    return large ? launch_cfg<float, 128, 128, 2, 2, E, TOut>(a, w, bias, bias_bf16, c, M, N, K, lda,  \
+                                                               ldw, ldc, vec_store, s)                \
+                 : launch_cfg<float, 64, 64, 2, 2, E, TOut>(a, w, bias, bias_bf16, c, M, N, K, lda,    \
+                                                             ldw, ldc, vec_store, s);
+  switch (epi) {
+    CGPT_F32_CASE(CGPT_EPI_NONE)
+    CGPT_F32_CASE(CGPT_EPI_BIAS)
+    CGPT_F32_CASE(CGPT_EPI_BIAS_GELU)
+    CGPT_F32_CASE(CGPT_EPI_BIAS_RESID)
+    default: return CGPT_EINVAL;
+  }
+#undef CGPT_F32_CASE
+}
+
 template <typename TIn, typename TOut>
 static int launch_epi(int epi, int tile, const void* a, const void* w, const void* bias,
                       bool bias_bf16, void* c, int M, int N, int K, int64_t lda, int64_t ldw,
@@ -1879,8 +1922,7 @@ static int launch_epi(int epi, int tile, const void* a, const void* w, const voi
 #undef CGPT_EL_CASE
   }
   if constexpr (sizeof(TIn) == 4) {
-    return launch_gemm_split(epi, tile, a, w, bias, bias_bf16, c, sizeof(TOut) == 2, M, N, K, lda, ldw,
-                             ldc, vec_store, s);
+    return CGPT_EINVAL;  // launch_f32
   } else {
     switch (epi) {
       case CGPT_EPI_BIAS_RESID:
@@ -2021,7 +2063,6 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
   const bool f32_far = !bf16 && !f16 && !gemm_split_ok(lda, ldw);
   if (epilogue == CGPT_EPI_BIAS_RESID) {
     if (tile == CGPT_TILE_SKINNY) return CGPT_EINVAL;  // not a skinny epilogue
-    el = el || f32_far;
     // launch_resid picks the kernel (tile: a preference; an id it does not
     // take for these dtypes, in or out of the tile tables, means TILE_AUTO).
     if (el) {
@@ -2041,7 +2082,8 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
       return launch_resid<bf16_t, bf16_t>(tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, s);
     if (bf16)
       return launch_resid<bf16_t, float>(tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, s);
-    return launch_gemm_split(epilogue, tile, a, w, bias, bb, c, out16, m, n, k, lda, ldw, ldc, vec_store, s);
+    return out16 ? launch_f32<bf16_t>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, f32_far, s)
+                 : launch_f32<float>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, f32_far, s);
   }
   if (tile != CGPT_TILE_AUTO && tile != CGPT_TILE_SKINNY && (tile < 0 || tile >= nt))
     return CGPT_EINVAL;
@@ -2055,7 +2097,6 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
     return launch_gemm_skinny(bf16, epilogue, a, w, bias, bb, c, out16, m, n, k, lda, ldw, ldc,
                               nullptr, 0, nullptr, 0, s);
   }
-  el = el || f32_far;
   if (el) tile = 0;  // the element-load kernel has one tile
   if (tile == CGPT_TILE_AUTO && (bf16 || f16)) {
     const bool kgroup = gemm_kgroup_ok(M, N, K, lda, ldw, ldc, c, out16);
@@ -2089,6 +2130,9 @@ extern "C" int cgpt_gemm(const void* a, const void* w, const void* bias, void* c
     return launch_epi<bf16_t, bf16_t>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, el, s);
   if (bf16)
     return launch_epi<bf16_t, float>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, el, s);
+  if (!el)
+    return out16 ? launch_f32<bf16_t>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, f32_far, s)
+                 : launch_f32<float>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, f32_far, s);
   if (!out16)
     return launch_epi<float, float>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, el, s);
   return launch_epi<float, bf16_t>(epilogue, tile, a, w, bias, bb, c, m, n, k, lda, ldw, ldc, vec_store, el, s);

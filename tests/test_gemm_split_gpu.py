@@ -119,6 +119,29 @@ def test_split_tiny_rows(gpu, scale):
     assert row.max() < 4 * 2.0 ** -24 * math.sqrt(k), row.max()
 
 
+# The fp32 MFMA kernel of short K, at the edges of its rule, its tiles (64x64,
+# 128x128 from 512 of them) and 4-wide stores, and for rows 2^22 apart.
+@pytest.mark.parametrize("m,n,k", [(1, 1, 4), (16, 130, 64), (65, 33, 44), (65, 64, 16), (520, 577, 48),
+                                   (1025, 301, 60), (4095, 2051, 64), (8191, 1153, 32), (100, 50257, 20)])
+def test_short_k(gpu, m, n, k):
+    test_split_shapes(gpu, m, n, k)
+    a, w, b = randn(gpu, m, k, seed=1), randn(gpu, n, k, seed=2, scale=0.2), randn(gpu, n, seed=3)
+    ref = a.double() @ w.double().t() + b.double()
+    check(run(gpu, a, w, b, _lib.EPI_BIAS_GELU), a, w, torch.nn.functional.gelu(ref, approximate="tanh"))
+    out = run(gpu, a, w, b, _lib.EPI_BIAS, BF16)
+    assert ((out.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("epi", [_lib.EPI_BIAS, _lib.EPI_BIAS_RESID])
+def test_rows_far_apart(gpu, epi):
+    m, n, k = 70, 90, 100
+    a = torch.empty(70, 1 << 22, device=gpu)[:, :k]
+    a.copy_(randn(gpu, m, k, seed=1))
+    w, b, c = randn(gpu, n, k, seed=2), randn(gpu, n, seed=3), randn(gpu, m, n, seed=4)
+    ref = a.double() @ w.double().t() + b.double() + (c.double() if epi == _lib.EPI_BIAS_RESID else 0)
+    check(run(gpu, a, w, b, epi, c=c), a, w, ref)
+
+
 # Small elements in rows that hold ordinary ones too, each against a partner of
 # the inverse scale; e < 0: in W.  Products are of order one, so the bound of
 # `check` holds with the sum of their sizes for the norms.
