@@ -363,13 +363,18 @@ static int launch_split_epi(int tile, const void* a, const void* w, const void* 
 //    epilogue overlaps nothing, so scalar stores go to the smaller tiles:
 //    1000 x 50257 x 768 732 -> 509 with 128x128 (256x256 566);
 //  * 128x128, three blocks a CU, from 2.5 of them a CU: 4096 x 3072 x 768
-//    201 -> 123;
+//    201 -> 123; of one row of tiles and K up to 256 from one a CU: 100 x 50257 x
+//    128 30.2 (128x64 34.5), 70 x 50304 x 256 26.0 (32.8), x 384 the same;
 //  * fewer, and long K: 128x128 with two K groups, 4096 x 768 x 3072 173 -> 123
 //    (one group 156), 1500 x 1600 x 6400 351 -> 220 (128x64 239);
 //  * 128x64 with two K groups: 4096 x 2304 x 768 138 -> 96, 4096 x 768 x 768
-//    48 -> 38 (128x128 with two 39), 520 x 3072 x 768 37 -> 24;
+//    48 -> 38 (128x128 with two 39), 520 x 3072 x 768 37 -> 24,
+//    and whenever 64x64 tiles, one block a CU, would need a second round:
+//    1500 x 768 x 768 24.2 (64x64 29.8), 7000 x 192 x 192 11.8 (16.9);
 //  * 64x64 with four K groups from 5/8 of a tile a CU: 200 x 3072 x 768
-//    24 -> 15 (128x64 21, 32x32 18);
+//    24 -> 15 (128x64 21, 32x32 18), and when 32x32 tiles, two blocks a CU, would
+//    need a second round: 1500 x 384 x 768 16.0 (32x32 20.3), x 128 7.5 (11.4);
+//    up to K = 128 when they are more than one a CU: 900 x 384 x 96 7.0 (7.8);
 //  * 32x32, a wave a K group: eight groups while that is one round of blocks,
 //    87 x 768 x 3072 77 -> 20 (64x64 38), 87 x 2304 x 768 23 -> 8.8; four
 //    beyond (two blocks a CU), 65 x 3072 x 768 22 -> 12.2 (eight: 15); of
@@ -384,11 +389,12 @@ static int split_tile(int M, int N, int K, bool vec_store) {
   const int64_t t256 = tiles(256, 256), rounds = (t256 + cus - 1) / cus;
   if (t256 >= cus && vec_store && 4 * t256 >= 3 * rounds * cus) return k256x256;
   const int64_t t128 = tiles(128, 128);
-  if (2 * t128 >= 5 * cus) return k128x128;
+  if (2 * t128 >= 5 * cus || (M <= 128 && t128 > cus && K <= 256)) return k128x128;
   if (2 * t128 >= cus && K >= 1536) return k128x128k2;
-  if (8 * tiles(128, 64) >= 6 * cus) return k128x64k2;
-  if (8 * tiles(64, 64) >= 5 * cus) return k64x64k4;
-  return tiles(32, 32) <= cus ? k32x32k8 : k32x32k4;
+  const int64_t t64 = tiles(64, 64), t32 = tiles(32, 32);
+  if (8 * tiles(128, 64) >= 6 * cus || t64 > cus) return k128x64k2;
+  if (8 * t64 >= 5 * cus || t32 > (K <= 128 ? 1 : 2) * cus) return k64x64k4;
+  return t32 <= cus ? k32x32k8 : k32x32k4;
 }
 
 bool gemm_split_ok(int64_t lda, int64_t ldw) { return lda < (1 << 22) && ldw < (1 << 22); }

@@ -119,6 +119,34 @@ def test_split_tiny_rows(gpu, scale):
     assert row.max() < 4 * 2.0 ** -24 * math.sqrt(k), row.max()
 
 
+# A shape for each tile of the size rule, K past the fp32 MFMA kernel's and ending
+# within a stage.
+TILES = [(65, 33, 68), (2700, 192, 132), (300, 1000, 84), (1500, 384, 76), (1500, 768, 84), (100, 38400, 72),
+         (2049, 5121, 76), (1409, 1537, 1540), (4090, 4092, 84)]
+
+
+@pytest.mark.parametrize("m,n,k", TILES)
+def test_split_tiles(gpu, m, n, k):
+    test_split_shapes(gpu, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", TILES)
+def test_split_tiles_non_finite(gpu, m, n, k):
+    """A NaN, infinities and values past the split's range, in single rows."""
+    a, w, b = randn(gpu, m, k, seed=1), randn(gpu, n, k, seed=2), randn(gpu, n, seed=3)
+    a[m - 1, k - 1], a[m // 2, 3], w[n - 1, k - 2] = math.nan, math.inf, -math.inf
+    a[3, 5] = 3.4e38
+    w[:, 5] *= 1e-3
+    ref = (a.double() @ w.double().t() + b.double()).float()
+    out = run(gpu, a, w, b, _lib.EPI_BIAS)
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(out[inf], ref[inf])
+    fin = torch.isfinite(ref)
+    size = a.double().nan_to_num(0, 0, 0).abs() @ w.double().nan_to_num(0, 0, 0).abs().t() + 1.0
+    assert ((out.double() - ref.double()).abs()[fin] / size[fin]).max() < 1e-6
+
+
 # The fp32 MFMA kernel of short K, at the edges of its rule, its tiles (64x64,
 # 128x128 from 512 of them) and 4-wide stores, and for rows 2^22 apart.
 @pytest.mark.parametrize("m,n,k", [(1, 1, 4), (16, 130, 64), (65, 33, 44), (65, 64, 16), (520, 577, 48),
@@ -146,8 +174,7 @@ def test_rows_far_apart(gpu, epi):
 # the inverse scale; e < 0: in W.  Products are of order one, so the bound of
 # `check` holds with the sum of their sizes for the norms.
 @pytest.mark.parametrize("e", [-125, -115, -100, -80, 80, 100, 106, 115, 125])
-@pytest.mark.parametrize("m,n,k", [(97, 31, 64), (300, 1000, 36), (200, 3000, 52), (513, 3100, 100),
-                                   (1409, 1537, 1540), (2049, 5121, 32), (4095, 4100, 28)])
+@pytest.mark.parametrize("m,n,k", TILES + [(300, 1000, 36)])
 def test_split_inverse_scales(gpu, m, n, k, e):
     a, w = randn(gpu, m, k, seed=1), randn(gpu, n, k, seed=2)
     a[:, 1::2] *= 2.0 ** -e
@@ -163,7 +190,7 @@ def test_split_inverse_scales(gpu, m, n, k, e):
 @pytest.mark.parametrize("scale", [1e-38, 1e-42, 1e-44])
 def test_split_smallest_values(gpu, scale):
     """Small and subnormal values beside ordinary ones that meet zeros."""
-    m, n, k = 100, 90, 64
+    m, n, k = 100, 90, 72
     a, w = randn(gpu, m, k, seed=1), randn(gpu, n, k, seed=2) * 1e30
     a[:, ::2] *= scale
     w[:, 1::2] = 0.0
