@@ -1755,6 +1755,11 @@ static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, boo
 //    (24 x 768 x 3072 23.2 -> 19.3, but 24 x 50304 x 768 59 -> 66) or K is
 //    short (24 x 256 x 256 4.8 -> 5.6).  Up to 16 rows the skinny kernel's plain
 //    fp32 MFMAs cost less than splitting the weights: 16 x 2304 x 768 8.0 against 9.0.
+//    Above 32 rows N of more than half a column tile of 32 a CU and at most one
+//    stays with it, up to 48 rows or short of K = 1600: the skinny kernel has one
+//    round of blocks there and the 64x64 tiles fill half the CUs (33 x 5120 x 256
+//    6.0 against 8.5, 64 x 5120 x 1280 23.2 against 24.9, 33 x 8192 x 6400 74
+//    against 81; 64 x 5120 x 1600 26.5 against 26.1, 40 x 12288 x 512 18.1 / 14.1).
 static bool skinny_bf16(int64_t M, int64_t N, int64_t K, bool wide_tile, bool kgroup) {
   if (M > 64) return false;
   if (N >= kWideN) return M <= 32 || !wide_tile;
@@ -1764,6 +1769,8 @@ static bool skinny_bf16(int64_t M, int64_t N, int64_t K, bool wide_tile, bool kg
 static bool skinny_f32(int64_t M, int64_t N, int64_t K, bool far) {
   if (M > 64) return false;
   if (far || K < 256) return true;
+  const int64_t cus = num_cus();
+  if (M > 32 && N > 16 * cus && N <= 32 * cus && (M <= 48 || K < 1600)) return true;
   return M <= (N < kWideN && K >= 512 ? 16 : 32);
 }
 

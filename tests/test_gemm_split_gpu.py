@@ -125,6 +125,13 @@ TILES = [(65, 33, 68), (2700, 192, 132), (300, 1000, 84), (1500, 384, 76), (1500
          (2049, 5121, 76), (1409, 1537, 1540), (4090, 4092, 84)]
 
 
+# 33 to 64 rows on either side of the skinny kernel's band of N.
+@pytest.mark.parametrize("m,n,k", [(33, 4096, 256), (33, 4100, 256), (64, 8192, 260), (48, 8196, 260),
+                                   (49, 4104, 1600), (49, 4104, 1596)])
+def test_skinny_band(gpu, m, n, k):
+    test_split_shapes(gpu, m, n, k)
+
+
 @pytest.mark.parametrize("m,n,k", TILES)
 def test_split_tiles(gpu, m, n, k):
     test_split_shapes(gpu, m, n, k)
