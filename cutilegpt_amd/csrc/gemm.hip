@@ -1746,7 +1746,9 @@ static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, boo
 //    64 x 768 x 3072 19.5 -> 8.1, 32 x 1600 x 6400 31.6 -> 12.7,
 //    64 x 2304 x 768 8.1 -> 5.2; one row 1 x 768 x 3072 10.3 -> 7.8,
 //    1 x 2304 x 768 5.0 -> 4.9.  Two k64 steps are the least that gives two of
-//    the groups work.  Wide N (the LM heads) is weight streaming, which the
+//    the groups work; up to 16 rows of at most 24 KB of weights the groups'
+//    exchange costs more than the chains (in the caches: 8 x 48 x 192 2.7 against
+//    3.2, 16 x 64 x 128 2.8 against 3.2, 8 x 128 x 128 the same).  Wide N (the LM heads) is weight streaming, which the
 //    skinny kernel does at 22.9 us for 32 x 50304 x 768 (tiles 26 to 34); above
 //    32 rows its accumulators leave it too few loads in flight: 64 rows
 //    44.9 -> 28.4.
@@ -1763,7 +1765,7 @@ static int auto_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi, boo
 static bool skinny_bf16(int64_t M, int64_t N, int64_t K, bool wide_tile, bool kgroup) {
   if (M > 64) return false;
   if (N >= kWideN) return M <= 32 || !wide_tile;
-  return !kgroup || K < 128;
+  return !kgroup || K < 128 || (M <= 16 && N * K <= 12288);
 }
 
 static bool skinny_f32(int64_t M, int64_t N, int64_t K, bool far) {

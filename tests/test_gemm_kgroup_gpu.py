@@ -118,3 +118,10 @@ def test_one_row_view(gpu, row, width, dtype):
     # 16 bits: one rounding of the output; fp32: sqrt(768) roundings of the running sum
     tol = {F32: 2.0 ** -18, F16: 2.0 ** -10, BF16: 2.0 ** -7}[dtype]
     assert (out.double() - ref[row:row + 1]).abs().max() <= tol * ref.abs().max()
+
+
+# On either side of the skinny kernel's small weights (12288 of them, 16 rows).
+@pytest.mark.parametrize("m,n,k", [(1, 96, 128), (1, 100, 128), (16, 64, 192), (16, 68, 192), (17, 64, 192),
+                                   (8, 4, 3072), (8, 8, 3072)])
+def test_few_small_weights(gpu, m, n, k):
+    test_kgroup_shapes(gpu, m, n, k, BF16)
