@@ -1695,7 +1695,8 @@ static int cheapest_tile(int M, int N, int K, int64_t lda, int64_t ldw, int epi,
 // among them.  The CUs drift apart over many rounds and share the last one
 // better than predicted: heads with less than 2.5% to gain ran 0.97 to 1.03
 // times as fast (4096 x 50304 x 768, 0.8% predicted, 342 -> 352), those above
-// it 1.01 to 1.18.  Narrower products gained and lost (0.94 to 1.07).
+// it 1.01 to 1.18 up to eight rounds and 0.97 to 1.04 beyond (3000 x 50304 x 768,
+// 9.2 rounds, 1.03; 3300 x 50304 x 1600, one tile past ten, 0.97).  Narrower products gained and lost (0.94 to 1.07).
 static int64_t whole_round_columns(int tile, int M, int N, int K, int64_t lda, int64_t ldw, int epi,
                                    bool kgroup) {
   const TileCost* t = kTileCosts;
